@@ -160,6 +160,41 @@ def test_load_quant_byte_exact_and_usable(gpu, dtype, k, n):
     assert_close(y.cpu().numpy(), O.reference_matmul(dtype, x, ref, 1, n, k)[0], what="load_quant → GEMV")
 
 
+def random_bytes(dtype, n_blocks, seed):
+    """synth_blocks with scales of every kind in every 11th block (uniform f16 bits: exponent 31, subnormals,
+    zeros of either sign among them) and all-zero blocks."""
+    be, bb = GEOM[dtype]
+    raw = synth_blocks(dtype, n_blocks, seed).reshape(n_blocks, bb).copy()
+    rng = np.random.default_rng(seed)
+    some = raw[::11]
+    some[:] = rng.integers(0, 256, some.shape, dtype=np.uint8)
+    raw[5::17] = 0
+    return raw.ravel()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("k,n,where", [(256, 256, "apart"), (512, 768, "apart"), (768, 512, "apart"),
+                                       (256, 512, "shifted"), (256, 256, "odd"), (512, 256, "in place")])
+def test_load_quant_whole_super_blocks(gpu, dtype, k, n, where):
+    """n and k multiples of 256 take the one-pass tile kernel, byte for byte what the three passes give: one tile,
+    several each way, every kind of block scale; a source off its 16-byte alignment and a destination over the
+    source still give the same bytes."""
+    torch = gpu
+    L = A.lib()
+    be, bb = GEOM[dtype]
+    raw = random_bytes(dtype, k * n // be, 7 + k + n + dtype)
+    ws = torch.empty(L.aeth_load_quant_ws_bytes(k, n), dtype=torch.uint8, device="cuda")
+    src = torch.zeros(raw.size + 16, dtype=torch.uint8, device="cuda")
+    at = {"shifted": 2, "odd": 1}.get(where, 0)
+    src[at:at + raw.size] = to_dev(torch, raw)
+    out = src if where == "in place" else torch.full((raw.size + 16,), 0xA5, dtype=torch.uint8, device="cuda")
+    A.check(L.aeth_load_quant(dtype, src.data_ptr() + at, k, n, out.data_ptr() + at, ws.data_ptr(), None), "load_quant")
+    torch.cuda.synchronize()
+    got, ref = out.cpu().numpy()[at:at + raw.size], load_quant_oracle(dtype, raw, k, n)
+    bad = np.flatnonzero(got != ref)
+    assert bad.size == 0, "dtype %d k=%d n=%d: %d bytes differ, first at %d" % (dtype, k, n, bad.size, bad[0])
+
+
 def test_requantize_and_load_quant_bad_arguments(gpu):
     L = A.lib()
     assert L.aeth_requantize(3, None, 1, 32, None, None) == A.AETH_EUNSUPPORTED
