@@ -809,6 +809,34 @@ def test_gguf_order_matmul_parity(gpu, dtype, m, n, k):
     assert_close(got_acc, ref + y0.reshape(m, n), what="gguf-order accumulate")
 
 
+@pytest.mark.parametrize("dtype", [Q2_K, Q3_K])
+@pytest.mark.parametrize("m,n,k", [(1, 256, 33), (1, 1280, 1), (1, 5120, 515), (2, 1024, 96), (4, 1280, 257),
+                                   (5, 512, 64), (9, 2304, 130)])
+def test_gguf_packed_kernel_edges(gpu, dtype, m, n, k):
+    """Whole blocks per input (n % 256 == 0): part-filled 1024-output units, batches and splits, 1 / 4 / 8 rows a
+    workgroup, uniformly random block bytes (scales of every exponent and sign). Each output is a chain of at most
+    ceil(k/8) + 1 fused multiply-adds per wave, a tree over the waves and an f64 sum over the splits, of the very
+    weights dequant.rs rounds: |error| <= (ceil(k/8) + 6)·2^-24·Σ|x·w|. A row holding an infinity gives the
+    reference's infinities and NaN."""
+    torch = gpu
+    be, bb = GEOM[dtype]
+    rng = np.random.default_rng(dtype + m + n + k)
+    raw = rng.integers(0, 256, n * k // be * bb, dtype=np.uint8)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[0, k // 2] = 0.0
+    w64 = O.dequant(dtype, raw, n * k).astype(np.float64).reshape(k, n)
+    w = make_weight(torch, dtype, n, k, raw)
+    got = gemv(torch, w, x, n, m).astype(np.float64)
+    bound = (-(-k // 8) + 6) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w64))
+    assert (np.abs(got - x.astype(np.float64) @ w64) <= bound).all()
+    x[m - 1, k - 1] = -np.inf
+    got = gemv(torch, w, x, n, m)[m - 1]
+    A.lib().aeth_weight_free(w)
+    with np.errstate(invalid="ignore"):
+        ref = -np.inf * w64[k - 1]  # the other terms are finite
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(got[~np.isnan(ref)], ref[~np.isnan(ref)])
+
+
 def test_gguf_order_zero_activation_skips_infinite_weights(gpu):
     """A zero activation skips its weight row even when that row holds an
     infinity (0·inf would be NaN): matmul_f32_gguf's `if scale != 0.0`."""
