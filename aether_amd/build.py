@@ -21,6 +21,7 @@ SOURCES = [
     "aeth_gemm_kq.hip",
     "aeth_gemm_q6k.hip",
     "aeth_gemm_q80.hip",
+    "aeth_gemm_f16.hip",
     "aeth_decode_ops.hip",
     "aeth_prefill.hip",
     "aeth_backend.hip",
@@ -46,6 +47,7 @@ EXTRA = {
     "aeth_gemm_kq.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "aeth_gemm_q6k.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "aeth_gemm_q80.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "aeth_gemm_f16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 COMMON = [

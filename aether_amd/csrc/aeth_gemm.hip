@@ -4,10 +4,10 @@
 // "Exact" mode on fp16 MFMA (v_mfma_f32_32x32x16_f16, fp32 accumulate):
 //  * A is split into two fp16 parts, A·2^-e = Ah + Al (Ah = fp16(A·2^-e),
 //    Al = fp16(A·2^-e − Ah)): 22 significant bits, f32-level. The power of two
-//    2^e is chosen per row so that the parts stay in fp16 range (e = 0 unless
-//    the row holds a value of magnitude ≥ 2^14); a shared exponent for several
-//    rows would push the lo parts of a small row next to a large one into fp16
-//    subnormals.
+//    2^e is chosen per row so that its largest value lies in [2^13, 2^14): the
+//    parts stay in fp16 range, and the lo parts of what matters to the row out of
+//    its subnormals (a row of 1e-4 unscaled keeps 13 bits; a shared exponent for
+//    several rows would do the same to a small row next to a large one).
 //  * Q4_K weights become exact fp16 integers w = q·sc (q ≤ 15, sc ≤ 63), so
 //    every MFMA product is exact and the K-sum is an f32 accumulation.
 //  * Per 256-element super-block b:  C += 2^e·(d_b·Σ A·(q·sc) − dmin_b·Σ_s m_s·S_s)
@@ -57,7 +57,7 @@
 #define G2_LOADS 6
 
 // ── activation prep (f32 A [m][k]; rows m..mp-1 read as zero). Writes
-//  * escale[r] = 2^e, e ≥ 0 the least with |A[r]·2^-e| < 2^14;
+//  * escale[r] = 2^e, e the least (from −100 on) with |A[r]·2^-e| < 2^14;
 //  * fragment (mt, ks, part) = 1 KiB at ((mt·nks + ks)·2 + part)·1024 bytes
 //    (nks = k/16): lane l holds row 32·mt + l%32 at k-positions
 //    16·ks + 8·(l/32) + perm4(i), i < 8, of A·2^-e, part 0 = hi, 1 = lo;
@@ -99,6 +99,7 @@ struct PrepArgs {
     int m, k;
     float* escale;
     _Float16 *frag, *Sh, *Sl;
+    int keep_inf;         // an infinite element: hi = ±Inf, lo = 0, the row's scale from its finite ones (F16 weights)
 };
 
 // 8 consecutive floats at p (16-byte aligned when AL16)
@@ -198,7 +199,10 @@ __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs
 #pragma unroll
         for (int t = 0; t < SPW; t++)
 #pragma unroll
-            for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(v[t][i]));
+            for (int i = 0; i < 8; i++) {
+                const float av = fabsf(v[t][i]);
+                mx = fmaxf(mx, P.keep_inf && av == INFINITY ? 0.0f : av);
+            }
     }
     mx = aeth_wave_max(mx);
     if (lane == 0) red[1][wv] = mx;
@@ -206,9 +210,9 @@ __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs
     mx = 0.0f;
 #pragma unroll
     for (int q = 0; q < WK; q++) mx = fmaxf(mx, red[1][PREP_ROWS * q + ri]);
-    int E = 0;
+    int E = 14;
     if (mx > 0.0f && isfinite(mx)) (void)frexpf(mx, &E);
-    const float esc = ldexpf(1.0f, E > 14 ? E - 14 : 0);
+    const float esc = ldexpf(1.0f, max(E - 14, -100));
     if (j == 0 && lane == 0) P.escale[r] = esc;
     const float inv = 1.0f / esc;  // a power of two: the products below are exact scalings
     const int tp = tid % (64 * PREP_ROWS);  // thread of the part's PREP_ROWS waves
@@ -253,7 +257,7 @@ __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs
                 const float tv = x[perm4(i)] * inv;
                 const _Float16 th = (_Float16)tv;
                 hi[i] = th;
-                lo[i] = (_Float16)(tv - (float)th);
+                lo[i] = P.keep_inf && fabsf(tv) == INFINITY ? (_Float16)0.0f : (_Float16)(tv - (float)th);
             }
             if (sl && gi < ng && (lane & 3) == 0) {  // gi < ng is uniform per four lanes (ng % 32 == 0)
                 const float sv = sum * inv * 0.03125f;
@@ -513,7 +517,7 @@ static void prep_launch(int spw, unsigned mp, hipStream_t s, const PrepArgs& P) 
 // The activation prep of the Q4_K and Q6_K GEMMs: A (or, with `in`, its producer's input) into
 // hi/lo fp16 MFMA fragments, sub-block sums and row scales in ws (the stream's scratch when null).
 static int gemm_prep(const float* d_a, int64_t m, int k, unsigned flags, const GemmIn* in, hipStream_t s, void* ws,
-                     size_t ws_bytes, _Float16*& frag, _Float16*& Sh, float*& esc) {
+                     size_t ws_bytes, _Float16*& frag, _Float16*& Sh, float*& esc, bool keep_inf = false) {
     const int mode = in ? in->mode : PREP_PLAIN;
     const int64_t mp = aeth_cdiv(m, G2_BM) * G2_BM;  // fragment rows: whole 64-row tiles
     if (mp > (1LL << 20) || mp * k > (1LL << 29)) return aeth_set_error(AETH_EINVAL, "gemm: m=%lld too large", (long long)m);
@@ -534,7 +538,7 @@ static int gemm_prep(const float* d_a, int64_t m, int k, unsigned flags, const G
     // registers per wave: its share of the row's steps, rounded up to 1, 2, 4 or 8 (past 8: chunks)
     const int share = (int)aeth_cdiv(aeth_cdiv(k, 512), PREP_WK);
     const int spw = share <= 1 ? 1 : share <= 2 ? 2 : share <= 4 ? 4 : 8;
-    const PrepArgs P{d_a, in ? in->norm_w : nullptr, in ? in->eps : 0.0f, (int)m, k, esc, frag, Sh, Sl};
+    const PrepArgs P{d_a, in ? in->norm_w : nullptr, in ? in->eps : 0.0f, (int)m, k, esc, frag, Sh, Sl, keep_inf ? 1 : 0};
     const unsigned pg = (unsigned)mp;  // fragment rows (whole 64-row tiles)
     if (mode == PREP_RMSNORM) prep_launch<true, false, PREP_RMSNORM>(spw, pg, s, P);
     else if (mode == PREP_SWIGLU) prep_launch<true, false, PREP_SWIGLU>(spw, pg, s, P);
@@ -787,6 +791,37 @@ int aeth_gemm_q80_launch(const aeth_weight* w, const float* d_a, int64_t m, floa
               (flags & AETH_MM_ACCUMULATE) ? 1 : 0, swo ? 1 : 0, P.ksplit, P.part, (int)(gn * G2_BN), P.t_full,
               P.tsplit};
     return aeth_gemm_q80_kq_launch(Q, s);
+}
+
+bool aeth_f16_gemm_rows(const aeth_weight* w, int64_t m) {
+    if (!w || w->dtype != AETH_DTYPE_F16 || w->order != AETH_ORDER_GGUF || w->special_scales) return false;
+    if (w->k % 32 != 0 || w->n % 4 != 0) return false;  // whole prep groups, four columns a lane
+    const int64_t mp = aeth_cdiv(m, G2_BM) * G2_BM;
+    // buffer offsets are 32-bit (a larger product takes k_col)
+    if (w->bytes >= INT32_MAX || mp * w->k * 4 >= INT32_MAX || mp > (1LL << 20)) return false;
+    // 4096 × 4096 at 12 / 32 / 64 rows: 30.7 / 31.6 / 33.3 µs here, 35.7 / 50.0 / 88.4 in k_col; below 32
+    // rows k_col's short f32 chains (1.3e-7 of a result against 1.6e-7 here) are also the more exact
+    return m >= 32;
+}
+
+int aeth_gemm_f16_launch(const aeth_weight* w, const float* d_a, int64_t m, float* d_c, unsigned flags, hipStream_t s,
+                         int64_t ldc) {
+    if (!aeth_f16_gemm_rows(w, m)) return aeth_set_error(AETH_EINVAL, "gemm f16: shape not taken (m=%lld)", (long long)m);
+    const int k = (int)w->k;
+    if (ldc <= 0) ldc = w->n;
+    const int64_t mp = aeth_cdiv(m, G2_BM) * G2_BM, gm = mp / G2_BM, gn = aeth_cdiv(w->n, G2_BN);
+    _Float16 *frag, *Sh;
+    float* esc;
+    // the dot-product mode does not exist for F16: its flag is ignored
+    int rc = gemm_prep(d_a, m, k, flags & ~AETH_MM_Q8_ACTIVATIONS, nullptr, s, nullptr, 0, frag, Sh, esc, true);
+    if (rc) return rc;
+    SplitPlan P;  // each wave keeps at least 16 slices, the 256 elements of a K-quant super-block
+    if ((rc = split_plan(s, gm, gn, k / 2048, false, P))) return rc;
+    const int c16 = ((uintptr_t)d_c & 15) == 0 && (ldc & 3) == 0;
+    F16Args Q{(const uint8_t*)frag, esc, w->p0, (int)m, (int)w->n, k, (int)mp, (int)gm, (int)gn, (int)(mp * k * 4),
+              (int)w->bytes, d_c, ldc, (flags & AETH_MM_ACCUMULATE) ? 1 : 0, 0, c16, P.ksplit, P.part,
+              (int)(gn * G2_BN), P.t_full, P.tsplit};
+    return aeth_gemm_f16_kernel_launch(Q, s);
 }
 
 bool aeth_gemm_fused_ok(const aeth_weight* w, int64_t m, int mode, const float* d_a, const float* norm_w) {

@@ -297,6 +297,26 @@ struct Q80Args {
 };
 int aeth_gemm_q80_kq_launch(const Q80Args& G, hipStream_t s);
 
+// Arguments of the F16 GEMM kernel (aeth_gemm_f16.hip): A as for KqArgs, W the [k][n] halves.
+struct F16Args {
+    const uint8_t* frag;   // A·2^-e as fp16 MFMA fragments (k_gemm_prep)
+    const float* escale;   // [mp]: 2^e
+    const uint8_t* w;
+    int m, n, k, mp;
+    int gm, gn;            // 64-row and 128-column tiles of C
+    int a_bytes, w_bytes;  // buffer extents (each < 2^31)
+    float* C;
+    int64_t ldc;
+    int accumulate;
+    int swiglu;            // 0
+    int c16;               // rows of C are 16-byte aligned
+    int ksplit;            // K split over workgroups: as Q6Args
+    float* part;
+    int pld;
+    int t_full = 0, tsplit = 1;  // tail split: as KqArgs
+};
+int aeth_gemm_f16_kernel_launch(const F16Args& G, hipStream_t s);
+
 // Grid of a K-split GEMM launch (see g2_work) and its second kernel (none without a split).
 template <class Args>
 unsigned g2_grid(const Args& G) {

@@ -104,11 +104,12 @@ int aeth_qmatmul_ld(const aeth_weight* w, const float* d_a, int64_t m, float* d_
     if (m > 1 && aeth_q5k_gemm_rows(w, m)) return aeth_gemm_q4k_launch(w, d_a, m, d_c, flags, s, ldc);  // Q5_K
     if (m > 1 && aeth_q6k_gemm_rows(w, m)) return aeth_gemm_q6k_launch(w, d_a, m, d_c, flags, s, ldc);  // Q6_K
     if (m > 1 && aeth_q80_gemm_rows(w, m)) return aeth_gemm_q80_launch(w, d_a, m, d_c, flags, s, ldc);  // Q8_0
+    if (m > 1 && aeth_f16_gemm_rows(w, m)) return aeth_gemm_f16_launch(w, d_a, m, d_c, flags, s, ldc);
     // the other block formats from a few hundred rows on: dequantized once, one DGEMM (instead
     // of the weight streamed once per row by the batched GEMV). Their dequantized
     // weights are finite (K-quant scales go through decode_d), so the SGEMM's
-    // 0·w terms equal matmul_f32_gguf's skipped rows; F32 / F16 weights, which may
-    // hold infinities, keep the kernels that skip zero activations as the reference does.
+    // 0·w terms equal matmul_f32_gguf's skipped rows; F32 weights and F16 ones holding
+    // infinities or NaN keep the kernels that skip zero activations as the reference does.
     // (a Q8_0 weight with a NaN or infinite block scale stays on the GEMV: dequantized, its
     // q = 0 entries become 0·Inf = NaN, where q8_0.rs multiplies the block's sum by d)
     if (m >= dequant_gemm_rows(w->dtype) && w->dtype != AETH_DTYPE_F32 && w->dtype != AETH_DTYPE_F16 &&

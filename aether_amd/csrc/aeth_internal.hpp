@@ -60,7 +60,7 @@ struct aeth_weight {
     uint8_t* base;
     uint8_t *p0, *p1, *p2, *p3;
     // planar weights: some block scale (Q8_0 d; Q4_K / Q5_K d or dmin; Q6_K d) has the f16
-    // exponent 31 (NaN / infinity bits), found when the bytes are laid out
+    // exponent 31 (NaN / infinity bits), found when the bytes are laid out; GGUF-order F16: some weight has
     int special_scales = 0;
 };
 
@@ -166,6 +166,11 @@ bool aeth_q80_gemm_fuses(const aeth_weight* w, int64_t m, int mode, const float*
 // aeth_q80_gemm_fuses.
 int aeth_gemm_q80_launch(const aeth_weight* w, const float* d_a, int64_t m, float* d_c, unsigned flags,
                          hipStream_t s, int64_t ldc = 0, const GemmIn* in = nullptr);
+// Whether m activation rows against GGUF-order F16 weight w take the F16 GEMM (aeth_gemm_f16.hip): every
+// weight finite, k a multiple of 32, n of 4, within the kernel's 32-bit buffer offsets, from 32 rows.
+bool aeth_f16_gemm_rows(const aeth_weight* w, int64_t m);
+int aeth_gemm_f16_launch(const aeth_weight* w, const float* d_a, int64_t m, float* d_c, unsigned flags, hipStream_t s,
+                         int64_t ldc = 0);
 // The runner's view of the three GEMMs: whether weight w takes producer `mode` in a GEMM
 // (Q4_K, Q6_K, Q8_0), whether its GEMM writes the SwiGLU output (Q4_K, Q8_0), and the launch.
 bool aeth_gemm_fused_ok(const aeth_weight* w, int64_t m, int mode, const float* d_a, const float* norm_w);

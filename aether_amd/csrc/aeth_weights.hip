@@ -211,7 +211,20 @@ __global__ void k_q5_gemm_bits(const uint8_t* __restrict__ raw, int64_t n, int64
             }
 }
 
-// Raw (GGUF-order or row) weights: the bytes as given, one allocation.
+// *flag set if some half of src has exponent 31 (n % 8 == 0: 16 bytes a thread and step, whole)
+__global__ void __launch_bounds__(256) k_f16_special(const uint4* __restrict__ src, int64_t n16, int* __restrict__ flag) {
+    bool any = false;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (int64_t)gridDim.x * 256) {
+        const uint4 v = src[i];
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 4; j++)  // the exponent plus one carries into the sign's place where it is all ones
+            any |= (((w[j] & 0x7C007C00u) + 0x04000400u) & 0x80008000u) != 0u;
+    }
+    if (any) atomicOr(flag, 1);
+}
+
+// Raw (GGUF-order or row) weights: the bytes as given, one allocation (and a flag past them).
 static int create_raw(int dtype, int order, int64_t n, int64_t k, const void* raw, int raw_is_device, hipStream_t s,
                       aeth_weight** out) {
     const int64_t bytes = aeth_weight_raw_bytes(dtype, order, n, k);
@@ -242,7 +255,8 @@ static int create_raw(int dtype, int order, int64_t n, int64_t k, const void* ra
     w->block_bytes = bb;
     w->nblk = bytes / bb;
     w->bytes = bytes;
-    hipError_t e = hipMalloc((void**)&w->base, (size_t)(bytes > 0 ? bytes : 256));
+    const int64_t flag_off = align256(bytes);
+    hipError_t e = hipMalloc((void**)&w->base, (size_t)(flag_off + 256));
     if (e != hipSuccess) {
         delete w;
         return aeth_set_error(AETH_ENOMEM, "aeth_weight_create: hipMalloc(%lld) failed: %s", (long long)bytes,
@@ -256,6 +270,29 @@ static int create_raw(int dtype, int order, int64_t n, int64_t k, const void* ra
         return aeth_set_error(AETH_EHIP, "aeth_weight_create: copy failed: %s", hipGetErrorString(e));
     }
     w->p0 = w->base;
+    // an F16 weight with an infinity or NaN keeps the kernel that skips zero activations (a tail of
+    // fewer than 8 halves counts as one: such shapes do not take the GEMM either)
+    if (dtype == AETH_DTYPE_F16 && order == AETH_ORDER_GGUF) {
+        int special = bytes % 16 != 0;
+        if (!special && bytes > 0) {
+            int* flag = (int*)(w->base + flag_off);
+            e = hipMemsetAsync(flag, 0, sizeof(int), s);
+            if (e == hipSuccess) {
+                const int64_t n16 = bytes / 16;
+                hipLaunchKernelGGL(k_f16_special, dim3((unsigned)std::min<int64_t>(aeth_cdiv(n16, 256), 2048)), dim3(256),
+                                   0, s, (const uint4*)w->base, n16, flag);
+                e = hipGetLastError();
+            }
+            if (e == hipSuccess) e = hipMemcpyAsync(&special, flag, sizeof(int), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipStreamSynchronize(s);
+            if (e != hipSuccess) {
+                hipFree(w->base);
+                delete w;
+                return aeth_set_error(AETH_EHIP, "aeth_weight_create: scan failed: %s", hipGetErrorString(e));
+            }
+        }
+        w->special_scales = special;
+    }
     *out = w;
     return AETH_OK;
 }

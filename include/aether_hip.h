@@ -135,8 +135,10 @@ AETH_API int aeth_load_quant(int dtype, const void* d_src, int64_t k, int64_t n,
  *     row count (Q2_K 40, Q3_K 32), then the weight dequantized once and one
  *     rocBLAS f64 DGEMM (also every K-quant product of the dot-product mode
  *     with k not a multiple of 256);
+ *   - m >= 32, GGUF-order F16 of finite values, k a multiple of 32: the exact-mode
+ *     fp16 MFMA GEMM;
  *   - F32 / F16 / Q2_K / Q3_K in GGUF order: the kernel of matmul_f32_gguf
- *     (dispatch.rs:541-574) for the rows not sent to the DGEMM.
+ *     (dispatch.rs:541-574) for the rows not sent to the GEMM or DGEMM.
  * Stream scratch: the GEMMs' activation fragments and split-K partials, the
  * GGUF-order kernel's partials, and the DGEMM's dequantized weight, f64
  * operands and partials live in buffers the library keeps per (device,

@@ -837,6 +837,53 @@ def test_gguf_packed_kernel_edges(gpu, dtype, m, n, k):
     assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(got[~np.isnan(ref)], ref[~np.isnan(ref)])
 
 
+@pytest.mark.parametrize("m,n,k", [(32, 4, 32), (33, 132, 96), (65, 300, 544), (64, 128, 4096), (130, 1028, 1056),
+                                   (300, 5124, 64)])
+def test_gemm_f16_tiles_scales_infinities(gpu, m, n, k):
+    """The F16 GEMM at tile remainders, K split 1 .. 8 ways over waves and workgroups, rows scaled 2^20 and 2^-12 and
+    a zero row, subnormal weights, accumulate and an output row off 16-byte alignment, against the f64 product.
+    The split of A leaves 2^-22 of a product (and 2^-39 of a row's maximum); the sum runs through k/8 products a wave
+    and a tree. A row holding an infinity gives the f32 sum's infinities and NaN; a weight holding one keeps the
+    kernel that skips zero activations."""
+    torch = gpu
+    L = A.lib()
+    rng = np.random.default_rng(m + n + k)
+    wh = (rng.standard_normal((k, n)) * 0.05).astype(np.float16)
+    wh[::7, ::3] = np.float16(3e-6)  # subnormal
+    wh[::5, 1::4] = 0
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[1] *= 2.0 ** 20
+    x[2] *= 2.0 ** -12
+    x[3] = 0.0
+    raw = wh.view(np.uint8).reshape(-1)
+    w = make_weight(torch, F16, n, k, raw)
+    w64, x64 = wh.astype(np.float64), x.astype(np.float64)
+    bound = (k / 16 + 24) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64)) + \
+        2.0 ** -37 * np.abs(x64).max(axis=1, keepdims=True) * np.abs(w64).sum(axis=0)
+    ref = x64 @ w64
+    assert (np.abs(gemv(torch, w, x, n, m) - ref) <= bound).all()
+    y0 = rng.standard_normal((m, n)).astype(np.float32)
+    yd = dev(torch, np.concatenate([np.zeros(1, np.float32), y0.ravel()]))
+    xd = dev(torch, x)
+    A.check(L.aeth_qmatmul(w, xd.data_ptr(), m, yd.data_ptr() + 4, A.MM_ACCUMULATE, None), "qmatmul")
+    torch.cuda.synchronize()
+    got = yd.cpu().numpy()[1:].reshape(m, n)
+    assert (np.abs(got - (ref + y0)) <= bound + 2.0 ** -24 * np.abs(ref + y0)).all()
+    x[m - 1, k - 1], x[m - 1, 0] = np.inf, 1e6
+    got = gemv(torch, w, x, n, m)
+    L.aeth_weight_free(w)
+    with np.errstate(invalid="ignore"):
+        inf = np.inf * w64[k - 1]
+    assert np.array_equal(np.isnan(got[m - 1]), np.isnan(inf)) and np.array_equal(got[m - 1][w64[k - 1] != 0], inf[w64[k - 1] != 0])
+    assert (np.abs(got[:m - 1] - ref[:m - 1]) <= bound[:m - 1]).all()
+    wh[k // 2, 0] = np.inf
+    x[:, k // 2] = 0.0
+    x[m - 1, k - 1] = 1.0
+    w = make_weight(torch, F16, n, k, wh.view(np.uint8).reshape(-1))
+    assert np.isfinite(gemv(torch, w, x, n, m)).all()
+    L.aeth_weight_free(w)
+
+
 def test_gguf_order_zero_activation_skips_infinite_weights(gpu):
     """A zero activation skips its weight row even when that row holds an
     infinity (0·inf would be NaN): matmul_f32_gguf's `if scale != 0.0`."""
