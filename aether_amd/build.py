@@ -22,6 +22,7 @@ SOURCES = [
     "aeth_gemm_q6k.hip",
     "aeth_gemm_q80.hip",
     "aeth_gemm_f16.hip",
+    "aeth_gemm_gq.hip",
     "aeth_decode_ops.hip",
     "aeth_prefill.hip",
     "aeth_backend.hip",
@@ -48,6 +49,7 @@ EXTRA = {
     "aeth_gemm_q6k.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "aeth_gemm_q80.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "aeth_gemm_f16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "aeth_gemm_gq.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 COMMON = [

@@ -81,6 +81,13 @@ void aeth_blas_release_stream(hipStream_t s) {
     }
 }
 
+int aeth_narrow_launch(const double* p, int64_t m, int64_t n, int parts, float* c, int64_t ldc, int accumulate,
+                       hipStream_t s) {
+    hipLaunchKernelGGL(k_narrow, dim3(grid_for(m * n)), dim3(256), 0, s, p, m, n, parts, c, ldc, accumulate);
+    AETH_LAUNCH_CHECK();
+    return AETH_OK;
+}
+
 int aeth_dequant_gemm_launch(const aeth_weight* w, const float* d_a, int64_t m, float* d_c, int64_t ldc,
                              unsigned flags, hipStream_t s) {
     int be, bb;
@@ -160,8 +167,5 @@ int aeth_dequant_gemm_launch(const aeth_weight* w, const float* d_a, int64_t m, 
         h, rows ? rocblas_operation_transpose : rocblas_operation_none, rocblas_operation_none, (int)n, (int)m, (int)kc,
         &alpha, W64, rows ? (int)kx : (int)n, rows ? kc : kc * n, A64, (int)kx, kc, &beta, P64, (int)n, m * n, parts);
     if (st != rocblas_status_success) return aeth_set_error(AETH_EHIP, "rocblas_dgemm failed (status %d)", (int)st);
-    hipLaunchKernelGGL(k_narrow, dim3(grid_for(m * n)), dim3(256), 0, s, P64, m, n, parts, d_c, ldc,
-                       (flags & AETH_MM_ACCUMULATE) ? 1 : 0);
-    AETH_LAUNCH_CHECK();
-    return AETH_OK;
+    return aeth_narrow_launch(P64, m, n, parts, d_c, ldc, (flags & AETH_MM_ACCUMULATE) ? 1 : 0, s);
 }

@@ -79,7 +79,7 @@ namespace {
 // (4096 × 4096: 0.15 ms, 4096 × 14336: 0.73 ms), the GEMV grows with m (≈ 2 µs per row
 // at 4096 × 4096). Measured crossovers (HIP events, rotated weight copies): Q6_K 4096 ×
 // 4096 ≈ 64 rows, 4096 × 14336 ≈ 80, 1024 × 4096 ≈ 136; Q8_0 ≈ 112; Q5_K ≈ 80; Q2_K ≈ 40
-// and Q3_K ≈ 32 (GGUF order). Q6_K rows of whole super-blocks and Q8_0 rows of whole blocks take
+// and Q3_K ≈ 32 (GGUF order, and there only blocks that straddle inputs: aeth_gemm_gq.hip takes the others). Q6_K rows of whole super-blocks and Q8_0 rows of whole blocks take
 // the Q6_K / Q8_0 GEMMs (aeth_gemm_q6k.hip, aeth_gemm_q80.hip) instead, from the row counts
 // aeth_q6k_gemm_rows / aeth_q80_gemm_rows give.
 int64_t dequant_gemm_rows(int dtype) {
@@ -104,6 +104,7 @@ int aeth_qmatmul_ld(const aeth_weight* w, const float* d_a, int64_t m, float* d_
     if (m > 1 && aeth_q5k_gemm_rows(w, m)) return aeth_gemm_q4k_launch(w, d_a, m, d_c, flags, s, ldc);  // Q5_K
     if (m > 1 && aeth_q6k_gemm_rows(w, m)) return aeth_gemm_q6k_launch(w, d_a, m, d_c, flags, s, ldc);  // Q6_K
     if (m > 1 && aeth_q80_gemm_rows(w, m)) return aeth_gemm_q80_launch(w, d_a, m, d_c, flags, s, ldc);  // Q8_0
+    if (m > 1 && aeth_gq_gemm_rows(w, m)) return aeth_gemm_gq_launch(w, d_a, m, d_c, flags, s, ldc);
     if (m > 1 && aeth_f16_gemm_rows(w, m)) return aeth_gemm_f16_launch(w, d_a, m, d_c, flags, s, ldc);
     // the other block formats from a few hundred rows on: dequantized once, one DGEMM (instead
     // of the weight streamed once per row by the batched GEMV). Their dequantized

@@ -171,6 +171,13 @@ int aeth_gemm_q80_launch(const aeth_weight* w, const float* d_a, int64_t m, floa
 bool aeth_f16_gemm_rows(const aeth_weight* w, int64_t m);
 int aeth_gemm_f16_launch(const aeth_weight* w, const float* d_a, int64_t m, float* d_c, unsigned flags, hipStream_t s,
                          int64_t ldc = 0);
+// Whether m activation rows against GGUF-order Q2_K / Q3_K weight w take the int8 GEMM (aeth_gemm_gq.hip):
+// whole blocks per input (n % 256 == 0), k at most 65536, more than 24 rows (8 or 16 of a large weight).
+bool aeth_gq_gemm_rows(const aeth_weight* w, int64_t m);
+int aeth_gemm_gq_launch(const aeth_weight* w, const float* d_a, int64_t m, float* d_c, unsigned flags, hipStream_t s,
+                        int64_t ldc = 0);
+// c = (float)Σ_q p[q] (+ c) over `parts` f64 products [m][n] (aeth_blas.cpp)
+int aeth_narrow_launch(const double* p, int64_t m, int64_t n, int parts, float* c, int64_t ldc, int accumulate, hipStream_t s);
 // The runner's view of the three GEMMs: whether weight w takes producer `mode` in a GEMM
 // (Q4_K, Q6_K, Q8_0), whether its GEMM writes the SwiGLU output (Q4_K, Q8_0), and the launch.
 bool aeth_gemm_fused_ok(const aeth_weight* w, int64_t m, int mode, const float* d_a, const float* norm_w);

@@ -131,10 +131,12 @@ AETH_API int aeth_load_quant(int dtype, const void* d_src, int64_t k, int64_t n,
  *     below that; Q5_K / Q6_K / Q8_0 products the GEMMs do not take (k not
  *     whole super-blocks / blocks, buffers past 32-bit offsets) run the
  *     row-batched GEMV up to 80 / 80 / 112 rows, then the DGEMM below;
- *   - m > 1, GGUF-order Q2_K / Q3_K: the row-batched GEMV up to a per-format
- *     row count (Q2_K 40, Q3_K 32), then the weight dequantized once and one
- *     rocBLAS f64 DGEMM (also every K-quant product of the dot-product mode
- *     with k not a multiple of 256);
+ *   - m > 1, GGUF-order Q2_K / Q3_K: the row-batched kernel up to 24 rows (Q3_K 8,
+ *     Q2_K 16 from 40 million weights on), then the int8 MFMA product; with n not
+ *     a multiple of 256 (blocks straddling inputs) up to a per-format row count
+ *     (Q2_K 40, Q3_K 32), then the weight dequantized once and one rocBLAS f64
+ *     DGEMM (also every K-quant product of the dot-product mode with k not a
+ *     multiple of 256);
  *   - m >= 32, GGUF-order F16 of finite values, k a multiple of 32: the exact-mode
  *     fp16 MFMA GEMM;
  *   - F32 / F16 / Q2_K / Q3_K in GGUF order: the kernel of matmul_f32_gguf

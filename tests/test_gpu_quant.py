@@ -837,6 +837,51 @@ def test_gguf_packed_kernel_edges(gpu, dtype, m, n, k):
     assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(got[~np.isnan(ref)], ref[~np.isnan(ref)])
 
 
+@pytest.mark.parametrize("dtype", [Q2_K, Q3_K])
+@pytest.mark.parametrize("m,n,k", [(25, 256, 64), (33, 512, 100), (64, 256, 37), (65, 768, 1001), (130, 256, 4100),
+                                   (300, 2048, 320), (17, 10240, 4096)])
+def test_gguf_int8_gemm_edges(gpu, dtype, m, n, k):
+    """The int8 product of GGUF-order Q2_K / Q3_K batches at row-tile, step and K-split remainders, uniformly random
+    block bytes (scales of every exponent and sign), rows scaled 2^30 and 2^-30 and a zero row, A off 16-byte
+    alignment, accumulate. Each A·d is an integer of 30 bits against the largest of its row and block column
+    (1.5 units lost at most), the sums exact: |error| <= 2^-24·|result| + k·128·1.5·2^-29·max|A|·max|d| (twice that
+    with Q2_K's mins). A row holding an infinity or NaN gives the f64 product's."""
+    torch = gpu
+    L = A.lib()
+    be, bb = GEOM[dtype]
+    rng = np.random.default_rng(dtype + m + n + k)
+    raw = rng.integers(0, 256, n * k // be * bb, dtype=np.uint8)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[1] *= np.float32(2.0 ** 30)
+    x[2] *= np.float32(2.0 ** -30)
+    x[3] = 0.0
+    w64 = O.dequant(dtype, raw, n * k).astype(np.float64).reshape(k, n)
+    at = (0, 2) if dtype == Q2_K else (108,)
+    dmax = max(abs(float(O.decode_d(int(v)))) for a in at
+               for v in np.unique(raw.reshape(-1, bb)[:, a:a + 2].copy().view(np.uint16)))
+    w = make_weight(torch, dtype, n, k, raw)
+    y0 = rng.standard_normal((m, n)).astype(np.float32)
+    xd, yd = dev(torch, np.concatenate([np.zeros(1, np.float32), x.ravel()])), dev(torch, y0)
+    A.check(L.aeth_qmatmul(w, xd.data_ptr() + 4, m, yd.data_ptr(), A.MM_ACCUMULATE, None), "qmatmul")
+    torch.cuda.synchronize()
+    x64 = x.astype(np.float64)
+    ref = x64 @ w64
+    lost = k * 128 * 1.5 * 2.0 ** -29 * np.abs(x64).max(axis=1, keepdims=True) * dmax * len(at)
+    # Q2_K's reference weights are each rounded to f32
+    lost = lost + (2.0 ** -24 * (np.abs(x64) @ np.abs(w64)) if dtype == Q2_K else 0.0)
+    assert (np.abs(yd.cpu().numpy() - (ref + y0)) <= 2.0 ** -24 * (np.abs(ref) + np.abs(ref + y0)) + lost).all()
+    got = gemv(torch, w, x, n, m)
+    assert (np.abs(got - ref) <= 2.0 ** -24 * np.abs(ref) + lost).all()
+    x[0, k // 3] = -np.inf
+    x[m - 1, 1] = np.nan
+    bad = gemv(torch, w, x, n, m)
+    L.aeth_weight_free(w)
+    with np.errstate(invalid="ignore"):
+        inf = -np.inf * w64[k // 3]
+    assert np.array_equal(np.isnan(bad[0]), np.isnan(inf)) and np.array_equal(bad[0][~np.isnan(inf)], inf[~np.isnan(inf)])
+    assert np.isnan(bad[m - 1]).all() and np.array_equal(bad[1:m - 1], got[1:m - 1])
+
+
 @pytest.mark.parametrize("m,n,k", [(32, 4, 32), (33, 132, 96), (65, 300, 544), (64, 128, 4096), (130, 1028, 1056),
                                    (300, 5124, 64)])
 def test_gemm_f16_tiles_scales_infinities(gpu, m, n, k):
