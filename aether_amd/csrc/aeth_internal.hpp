@@ -210,6 +210,7 @@ enum {
     AETH_SCRATCH_ARGMAX = 3,
     AETH_SCRATCH_DEQ = 4,   // dequantized f32 weight of a batched product (aeth_blas.cpp)
     AETH_SCRATCH_QACT = 5,  // Q8_0 activation blocks and their f32 values (same)
+    AETH_SCRATCH_PATTN = 7, // K and V of a prompt as fp16 fragments (aeth_prefill.hip)
     AETH_SCRATCH_SPLIT = 6, // partial output tiles of a GEMM split over K across workgroups (aeth_gemm.hip)
 };
 int aeth_stream_scratch(hipStream_t s, int use, size_t bytes, void** out);

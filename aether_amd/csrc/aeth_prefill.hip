@@ -19,6 +19,7 @@
 #include <string.h>
 
 #include "aeth_common.hpp"
+#include "aeth_gemm_common.hpp"
 #include "aeth_internal.hpp"
 #include "aeth_ops_internal.hpp"
 
@@ -475,6 +476,389 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill_mf(const float* __restr
     }
 }
 
+// ── Long prompts: the same attention on the fp16 matrix cores ─────────────
+// The f32 matrix cores run at a sixteenth of the fp16 rate. Here q, k, v and the
+// probabilities are each split into two fp16 parts, x·2^-e = hi + lo (22
+// significant bits), and a product takes three passes, lo·hi, hi·lo and hi·hi
+// (the dropped lo·lo is 2^-24 of it), on v_mfma_f32_32x32x16_f16: the error
+// against f64 is below the f32 kernel's (n = 1000 / 2000 / 4000: 1.7 / 1.8 / 1.9e-7
+// of a result against 1.9 / 2.3 / 2.7e-7).
+//  * k_attn_split lays K and V out once per call, per KV head and tile of 32
+//    keys, as MFMA fragments with one power of two each for the tile's K and V
+//    (32 KiB a tile; its exponents beside). Keys past the last are zero.
+//  * k_attn_prefill_sp: workgroup = 128 columns (128/G queries × G heads of a KV
+//    head, the query-block pair {p, last − p}); wave = 32 columns × every other
+//    key tile. A stage of two tiles (64 KiB) is loaded to LDS while the stage
+//    before it is used. Sᵀ = K·Qᵀ leaves a lane 16 keys of one column; V's
+//    fragments take their keys in that order, so the probabilities are the B
+//    operand of Oᵀ = Vᵀ·Pᵀ as they stand. Probabilities are taken against a
+//    maximum that may be 2^8 stale, and a tile's enter its product times a power
+//    of two of their column's largest, so that neither a flat row nor a tile far
+//    below the maximum has them in fp16's subnormals.
+// What bounds it: at n = 2000 (32 / 8 heads: 325 → 126 µs, 8 of it k_attn_split) the matrix cores are busy a third
+// of the time, 30 % of the waves' time goes to waits for LDS and the stage barrier, 37 % to dependencies. Not the
+// phases of a SIMD's two waves: an odd wave that multiplies its values a stage late took 138 µs, four
+// independent chains in place of two 153; without the stage loads it would take 115.
+// A KV head with an infinity or NaN among its keys or values takes a plain f32
+// loop (the split has no infinities).
+#define SP_TILE 32768  // bytes of a key tile's fragments: K [8 k-steps][hi, lo][1 KiB], V [4 d-tiles][2 halves][hi, lo][1 KiB]
+#define SP_BAD 0x7FFF  // exponent of a tile holding an infinity or NaN
+
+typedef _Float16 sp_h8 __attribute__((ext_vector_type(8)));
+typedef float sp_f16 __attribute__((ext_vector_type(16)));
+
+// 8 floats·2^-e → hi and lo
+__device__ __forceinline__ void sp_split(const float (&x)[8], float inv, sp_h8& hi, sp_h8& lo) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float v = x[i] * inv;
+        hi[i] = (_Float16)v;
+        lo[i] = (_Float16)(v - (float)hi[i]);
+    }
+}
+// e with |x|·2^-e < 2^14 for |x| <= mx (2^14 at most 2^100 away: the factors below stay normal)
+__device__ __forceinline__ int sp_exponent(float mx) {
+    int E = 14;
+    if (mx > 0.0f) (void)frexpf(mx, &E);
+    return max(E - 14, -100);
+}
+
+__global__ void __launch_bounds__(256) k_attn_split(const float* __restrict__ layer_kv, int n, int nkv, int64_t max_seq,
+                                                    int ntiles, uint8_t* __restrict__ frag, int2* __restrict__ exps) {
+    __shared__ float red[2][4];
+    __shared__ int bad;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int g = blockIdx.x % nkv, t = blockIdx.x / nkv, k0 = 32 * t;
+    const float* K = layer_kv + (int64_t)g * max_seq * 128;
+    const float* V = layer_kv + (int64_t)(nkv + g) * max_seq * 128;
+    if (tid == 0) bad = 0;
+    // K: k-steps w and w + 4, lane = key lane%32, d 16·ks + 8·(lane/32) + i. V: (d-tile, half) pairs w and w + 4,
+    // lane = d 32·dt + lane%32, element i = key 16·half + 8·(i/4) + 4·(lane/32) + i%4 (Sᵀ's result order)
+    float kx[2][8], vx[2][8], km = 0.0f, vm = 0.0f;
+    bool nf = false;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int ks = w + 4 * u, key = k0 + (lane & 31);
+        const float* src = K + (int64_t)min(key, n - 1) * 128 + 16 * ks + 8 * (lane >> 5);
+        const float4 a = *(const float4*)src, b = *(const float4*)(src + 4);
+        const float r[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        const int dt = ks >> 1, hf = ks & 1;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            kx[u][i] = key < n ? r[i] : 0.0f;
+            const int vk = k0 + 16 * hf + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+            const float x = V[(int64_t)min(vk, n - 1) * 128 + 32 * dt + (lane & 31)];
+            vx[u][i] = vk < n ? x : 0.0f;
+            nf |= !(fabsf(kx[u][i]) < INFINITY) || !(fabsf(vx[u][i]) < INFINITY);
+            km = fmaxf(km, fabsf(kx[u][i]));
+            vm = fmaxf(vm, fabsf(vx[u][i]));
+        }
+    }
+    km = aeth_wave_max(km);
+    vm = aeth_wave_max(vm);
+    __syncthreads();
+    if (nf) bad = 1;
+    if (lane == 0) {
+        red[0][w] = km;
+        red[1][w] = vm;
+    }
+    __syncthreads();
+    const int ek = sp_exponent(fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3])));
+    const int ev = sp_exponent(fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3])));
+    const float ki = ldexpf(1.0f, -ek), vi = ldexpf(1.0f, -ev);
+    uint8_t* dst = frag + ((int64_t)g * ntiles + t) * SP_TILE + lane * 16;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        sp_h8 hi, lo;
+        sp_split(kx[u], ki, hi, lo);
+        *(sp_h8*)(dst + (w + 4 * u) * 2048) = hi;
+        *(sp_h8*)(dst + (w + 4 * u) * 2048 + 1024) = lo;
+        sp_split(vx[u], vi, hi, lo);
+        *(sp_h8*)(dst + 16384 + (w + 4 * u) * 2048) = hi;
+        *(sp_h8*)(dst + 16384 + (w + 4 * u) * 2048 + 1024) = lo;
+    }
+    if (tid == 0) exps[g * ntiles + t] = bad ? make_int2(SP_BAD, SP_BAD) : make_int2(ek, ev);
+}
+
+// Rows of a KV head with an infinity or NaN in its cache: thread = (column tid/4, d [32·(tid%4), +32)), plain f32.
+template <int G>
+__device__ __noinline__ void sp_plain(const float* qkv, int64_t qkv_stride, const float* K, const float* V, int n, int nh,
+                                      int g, int q0, int window, float* out) {
+    const int cc = threadIdx.x >> 2, d0 = 32 * (threadIdx.x & 3), query = q0 + cc / G, head = g * G + cc % G;
+    if (query >= n) return;
+    const float* q = qkv + (int64_t)query * qkv_stride + (int64_t)head * 128;
+    const float scale = 1.0f / sqrtf(128.0f);
+    float m = -INFINITY, l = 0.0f, o[32] = {};
+    for (int t = window > 0 ? max(0, query - window + 1) : 0; t <= query; t++) {
+        float s = 0.0f;
+        for (int d = 0; d < 128; d++) s = fmaf(q[d], K[(int64_t)t * 128 + d], s);
+        s *= scale;
+        const float mn = fmaxf(m, s), al = mn == -INFINITY ? 1.0f : expf(m - mn);
+        const float p = mn == -INFINITY ? 0.0f : expf(s - mn);
+        l = l * al + p;
+        for (int d = 0; d < 32; d++) o[d] = o[d] * al + p * V[(int64_t)t * 128 + d0 + d];
+        m = mn;
+    }
+    for (int d = 0; d < 32; d++) out[(int64_t)query * nh * 128 + (int64_t)head * 128 + d0 + d] = o[d] * (1.0f / l);
+}
+
+template <int G>
+__global__ void __launch_bounds__(512, 2) k_attn_prefill_sp(const float* __restrict__ qkv, int64_t qkv_stride,
+                                                            const float* __restrict__ layer_kv,
+                                                            const uint8_t* __restrict__ frag,
+                                                            const int2* __restrict__ exps, int n, int nh, int nkv,
+                                                            int64_t max_seq, int ntiles, int window,
+                                                            float* __restrict__ out) {
+    constexpr int QB = 128 / G, PLD = 132;
+    constexpr float TH = 8.0f;  // log2: how stale a maximum may be
+    // two stages of two tiles (128 KiB), then the partial results [key parity][column][PLD] and their statistics
+    __shared__ __attribute__((aligned(1024))) char smem[2 * 128 * PLD * 4];
+    __shared__ float pm[2][128], pl[2][128];
+    __shared__ int pe[2][4];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), cg = w & 3, par = w >> 2;
+    const int c = 32 * cg + (lane & 31), hf = lane >> 5;
+    const int g = blockIdx.x % nkv, p = blockIdx.x / nkv;
+    const int nqb = (n + QB - 1) / QB;
+    const int head = g * G + c % G;
+    const uint8_t* fr = frag + (int64_t)g * ntiles * SP_TILE;
+    const int2* ex = exps + g * ntiles;
+    bool bad = false;
+    for (int t = lane; t < ntiles; t += 64) bad |= ex[t].x == SP_BAD;
+    bad = __any(bad);
+    const uint32_t sm0 = lds_addr(smem);
+    const float sl2 = 1.4426950408889634f / sqrtf(128.0f);  // scale · log2(e)
+    for (int pass = 0; pass < 2; pass++) {
+        const int qb = pass == 0 ? p : nqb - 1 - p;
+        if (pass == 1 && qb == p) break;  // the middle block of an odd count (uniform)
+        const int q0 = qb * QB, query = q0 + c / G;
+        if (bad) {
+            sp_plain<G>(qkv, qkv_stride, layer_kv + (int64_t)g * max_seq * 128,
+                        layer_kv + (int64_t)(nkv + g) * max_seq * 128, n, nh, g, q0, window, out);
+            continue;
+        }
+        const int kb_end = (min(q0 + QB, n) - 1) / 32;                           // last key tile, inclusive
+        const int kb_beg = window > 0 ? max(0, q0 - window + 1) / 32 : 0;        // first one any query sees
+        const int w_lo = q0 + 32 * cg / G, w_hi = q0 + (32 * cg + 31) / G;       // this wave's queries
+        // tiles kb_beg + 2·st + {0, 1} (past the last: the last again) → buffer st%2, 8 of the 64 KiB a wave
+        auto issue = [&](int st) {
+            const uint8_t* src = fr + (int64_t)min(kb_beg + 2 * st + (w >> 2), kb_end) * SP_TILE + (w & 3) * 8192 + lane * 16;
+            char* dst = smem + (st & 1) * 65536 + w * 8192;
+#pragma unroll
+            for (int i = 0; i < 8; i++) __builtin_amdgcn_global_load_lds(src + i * 1024, (lds_void*)(dst + i * 1024), 16, 0, 0);
+        };
+        issue(0);
+        sp_h8 qh[8], ql[8];
+        float fq;
+        {
+            const float* src = qkv + (int64_t)min(query, n - 1) * qkv_stride + (int64_t)head * 128 + 8 * hf;
+            float x[8][8], mx = 0.0f;
+#pragma unroll
+            for (int ks = 0; ks < 8; ks++) {
+                const float4 a = *(const float4*)(src + 16 * ks), b = *(const float4*)(src + 16 * ks + 4);
+                x[ks][0] = a.x; x[ks][1] = a.y; x[ks][2] = a.z; x[ks][3] = a.w;
+                x[ks][4] = b.x; x[ks][5] = b.y; x[ks][6] = b.z; x[ks][7] = b.w;
+#pragma unroll
+                for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(x[ks][i]));
+            }
+            mx = pa_max32(mx);
+            const int eq = sp_exponent(mx < INFINITY ? mx : 0.0f);  // an infinity makes the column NaN
+            const float inv = ldexpf(1.0f, -eq);
+#pragma unroll
+            for (int ks = 0; ks < 8; ks++) sp_split(x[ks], inv, qh[ks], ql[ks]);
+            fq = ldexpf(sl2, eq);
+        }
+        float m = -INFINITY, l = 0.0f;
+        int eo = -1000;  // the output's exponent: V tiles with a larger one raise it
+        sp_f16 o[4];
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) o[dt] = (sp_f16){};
+        const int nst = (kb_end - kb_beg) / 2 + 1;
+        sp_h8 ph[2], plo[2];  // the probabilities of a tile, hi and lo
+        float ve = 0.0f;      // and the scale of their product with its values against the output's
+        // o += Vᵀ·Pᵀ of the tile whose V is at vb. A tile's product forms apart, takes the tile's exponent and is added
+        // once: six roundings of a small sum and one of o, not six of o
+        auto values = [&](uint32_t vb) {
+            constexpr int LA = 2;  // fragments read ahead
+            sp_h8 f[LA + 1][2];
+            sp_f16 t4[2];
+#pragma unroll
+            for (int u = 0; u < LA; u++) {
+                f[u][0] = lds_b128h<0>(vb + u * 2048);
+                f[u][1] = lds_b128h<1024>(vb + u * 2048);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) {  // (d-tile u/2, key half u%2)
+                const int dt = u >> 1, c = u % (LA + 1);
+                if (u < 8 - LA) {
+                    f[(u + LA) % (LA + 1)][0] = lds_b128h<0>(vb + (u + LA) * 2048);
+                    f[(u + LA) % (LA + 1)][1] = lds_b128h<1024>(vb + (u + LA) * 2048);
+                    lgkm_wait<2 * LA>();
+                } else if (u == 6) {
+                    lgkm_wait<2>();
+                } else {
+                    lgkm_wait<0>();
+                }
+                pin(f[c][0]);
+                pin(f[c][1]);
+                sp_f16 x = (u & 1) ? t4[dt & 1] : (sp_f16){};
+                x = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[c][1], ph[u & 1], x, 0, 0, 0);
+                x = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[c][0], plo[u & 1], x, 0, 0, 0);
+                t4[dt & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[c][0], ph[u & 1], x, 0, 0, 0);
+                if ((u & 1) == 0 && dt > 0) o[dt - 1] += t4[(dt - 1) & 1] * ve;  // under this d-tile's products
+            }
+            o[3] += t4[1] * ve;
+        };
+        // Sᵀ of the tile whose K is at kb, and its probabilities
+        auto scores = [&](uint32_t kb, int t0, int2 e) {
+            sp_f16 s0[2] = {(sp_f16){}, (sp_f16){}}, s1 = (sp_f16){};  // hi·hi in two chains, the lo passes
+            constexpr int LA = 2;
+            sp_h8 f[LA + 1][2];
+#pragma unroll
+            for (int u = 0; u < LA; u++) {
+                f[u][0] = lds_b128h<0>(kb + u * 2048);
+                f[u][1] = lds_b128h<1024>(kb + u * 2048);
+            }
+#pragma unroll
+            for (int ks = 0; ks < 8; ks++) {
+                const int c = ks % (LA + 1);
+                if (ks < 8 - LA) {
+                    f[(ks + LA) % (LA + 1)][0] = lds_b128h<0>(kb + (ks + LA) * 2048);
+                    f[(ks + LA) % (LA + 1)][1] = lds_b128h<1024>(kb + (ks + LA) * 2048);
+                    lgkm_wait<2 * LA>();
+                } else if (ks == 6) {
+                    lgkm_wait<2>();
+                } else {
+                    lgkm_wait<0>();
+                }
+                pin(f[c][0]);
+                pin(f[c][1]);
+                s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[c][1], qh[ks], s1, 0, 0, 0);
+                s0[ks & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[c][0], qh[ks], s0[ks & 1], 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[c][0], ql[ks], s1, 0, 0, 0);
+            }
+            const float fs = ldexpf(fq, e.x);
+            float s[16], mx = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 16; r++) s[r] = ((s0[0][r] + s0[1][r]) + s1[r]) * fs;
+            if (!(t0 + 31 <= w_lo && t0 + 31 < n && (window <= 0 || t0 > w_hi - window))) {  // some key is masked (uniform)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int key = t0 + 8 * (r >> 2) + 4 * hf + (r & 3);
+                    if (!(key <= query && key < n && (window <= 0 || key > query - window))) s[r] = -INFINITY;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[r]);
+            mx = pa_max32(mx);
+            if (__any(mx > m + TH)) {  // uniform
+                const float mn = fmaxf(m, mx), al = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+                l *= al;
+#pragma unroll
+                for (int dt = 0; dt < 4; dt++) o[dt] *= al;
+                m = mn;
+            }
+            if (e.y > eo) {  // uniform
+                const float al = ldexpf(1.0f, max(eo - e.y, -250));
+#pragma unroll
+                for (int dt = 0; dt < 4; dt++) o[dt] *= al;
+                eo = e.y;
+            }
+            const float mo = m == -INFINITY ? 0.0f : m;  // every key masked so far: s − mo is −Inf
+            // the tile's largest probability of this column times 2^j lies in (2^12, 2^13]
+            const int j = mx == -INFINITY ? 0 : 13 - max((int)ceilf(mx - mo), -100);
+            const float fj = ldexpf(1.0f, j);
+            ve = ldexpf(1.0f, max(e.y - eo, -120) - j);
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                s[r] = __builtin_amdgcn_exp2f(s[r] - mo);
+                const float pv = s[r] * fj;
+                ph[r >> 3][r & 7] = (_Float16)pv;
+                plo[r >> 3][r & 7] = (_Float16)(pv - (float)ph[r >> 3][r & 7]);
+            }
+#pragma unroll
+            for (int h = 8; h >= 1; h /= 2)  // the tile's sum as a tree: one rounding of l a tile
+#pragma unroll
+                for (int r = 0; r < h; r++) s[r] += s[r + h];
+            l += s[0];
+        };
+        for (int st = 0; st < nst; st++) {
+            const int t = kb_beg + 2 * st + par, t0 = 32 * t;
+            vm_wait<0>();                 // this wave's part of stage st has landed
+            __builtin_amdgcn_s_barrier();  // and every wave's; the other stage's buffers are read
+            if (st + 1 < nst) issue(st + 1);
+            if (t > kb_end || t0 > w_hi || (window > 0 && t0 + 31 <= w_lo - window)) continue;  // nothing visible (uniform)
+            const uint32_t at = sm0 + (st & 1) * 65536 + par * 32768 + lane * 16;
+            scores(at, t0, ex[t]);
+            values(at + 16384);
+        }
+        __syncthreads();  // the stages are read: their LDS takes the partial results
+        float* po = (float*)smem + (par * 128 + c) * PLD;
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4)  // d = 32·dt + 2·r + 4·hf
+                *(float4*)(po + 32 * dt + 2 * r + 4 * hf) = make_float4(o[dt][r], o[dt][r + 1], o[dt][r + 2], o[dt][r + 3]);
+        l = pa_sum32(l);
+        if (hf == 0) {
+            pm[par][c] = m;
+            pl[par][c] = l;
+        }
+        if (lane == 0) pe[par][cg] = eo;
+        __syncthreads();
+        {  // merge the two key parities: thread → column tid/4, d 4·(tid%4) + 16·i
+            const int cc = tid >> 2, qq = q0 + cc / G, hh = g * G + cc % G;
+            const float m0 = pm[0][cc], m1 = pm[1][cc], M = fmaxf(m0, m1);
+            const float w0 = m0 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m0 - M);
+            const float w1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - M);
+            const float inv = 1.0f / (w0 * pl[0][cc] + w1 * pl[1][cc]);
+            const float a0 = ldexpf(w0 * inv, pe[0][cc >> 5]), a1 = ldexpf(w1 * inv, pe[1][cc >> 5]);
+            const float* x0 = (const float*)smem + cc * PLD;
+            const float* x1 = x0 + 128 * PLD;
+            if (qq < n) {
+                float* dst = out + (int64_t)qq * nh * 128 + (int64_t)hh * 128;
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const int d = 4 * (tid & 3) + 16 * i;
+                    const float4 u = *(const float4*)(x0 + d), v = *(const float4*)(x1 + d);
+                    *(float4*)(dst + d) = make_float4(a0 * u.x + a1 * v.x, a0 * u.y + a1 * v.y, a0 * u.z + a1 * v.z,
+                                                      a0 * u.w + a1 * v.w);
+                }
+            }
+        }
+        __syncthreads();  // LDS is reused by the second query block
+    }
+}
+
+// The split form where it is the faster one: its workgroups, one per pair of 128/G-query blocks and KV head, have to
+// fill enough of the chip. µs here and on the f32 kernel, 32 / 8 heads: n = 512 (64 workgroups) 41.6 / 37.3, 640 (80)
+// 48.0 / 59.6, 768 54 / 69.6, 1000 66 / 109, 2000 126 / 330, 4000 466 / 1318; 16 / 8 heads, n = 1000 (64) 62 / 57.
+// It needs a scratch of 32 KiB per KV head and 32 keys, the stream's own; under graph capture, where that could not grow
+// and a recorded address would not outlive a later growth, and where there is no memory for it, the f32 kernel runs.
+template <int G>
+static bool attn_split_launch(const float* qkv, int64_t stride, const float* layer_kv, int64_t n, int64_t nh, int64_t nkv,
+                              int64_t max_seq, int win, float* out, hipStream_t s, int* rc) {
+    *rc = AETH_OK;
+    const int64_t nqb = aeth_cdiv(n, 128 / G), wgs = nkv * aeth_cdiv(nqb, 2), nt = aeth_cdiv(n, 32);
+    if (wgs < 80) return false;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return false;
+    const int64_t fb = nkv * nt * SP_TILE;
+    void* ws = nullptr;
+    if (aeth_stream_scratch(s, AETH_SCRATCH_PATTN, (size_t)(fb + nkv * nt * sizeof(int2)), &ws) != AETH_OK) {
+        (void)hipGetLastError();
+        return false;
+    }
+    int2* ex = (int2*)((uint8_t*)ws + fb);
+    hipLaunchKernelGGL(k_attn_split, dim3((unsigned)(nkv * nt)), dim3(256), 0, s, layer_kv, (int)n, (int)nkv, max_seq, (int)nt,
+                       (uint8_t*)ws, ex);
+    hipLaunchKernelGGL(k_attn_prefill_sp<G>, dim3((unsigned)wgs), dim3(512), 0, s, qkv, stride, layer_kv, (const uint8_t*)ws, ex,
+                       (int)n, (int)nh, (int)nkv, max_seq, (int)nt, win, out);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) *rc = aeth_set_error(AETH_EHIP, "prefill attention: launch failed: %s", hipGetErrorString(e));
+    return true;
+}
+
 int aeth_attn_prefill_launch(const float* qkv, int64_t stride, const float* layer_kv, int64_t n, int64_t nh,
                              int64_t nkv, int64_t hd, int64_t max_seq, int64_t window, float* out, hipStream_t s) {
     if (n <= 0) return AETH_OK;
@@ -485,6 +869,12 @@ int aeth_attn_prefill_launch(const float* qkv, int64_t stride, const float* laye
     static const bool force_valu = getenv("AETH_PREFILL_ATTN") && !strcmp(getenv("AETH_PREFILL_ATTN"), "valu");
     const int64_t G = nh / nkv;
     if (!force_valu && (G == 1 || G == 2 || G == 4 || G == 8)) {
+        int rc;
+        if (G == 1 ? attn_split_launch<1>(qkv, stride, layer_kv, n, nh, nkv, max_seq, win, out, s, &rc)
+            : G == 2 ? attn_split_launch<2>(qkv, stride, layer_kv, n, nh, nkv, max_seq, win, out, s, &rc)
+            : G == 4 ? attn_split_launch<4>(qkv, stride, layer_kv, n, nh, nkv, max_seq, win, out, s, &rc)
+                     : attn_split_launch<8>(qkv, stride, layer_kv, n, nh, nkv, max_seq, win, out, s, &rc))
+            return rc;
         const int64_t nqb = aeth_cdiv(n, 16 / G);
         const dim3 grid((unsigned)(nkv * aeth_cdiv(nqb, 2)));
         if (G == 1) hipLaunchKernelGGL(k_attn_prefill_mf<1>, grid, dim3(256), 0, s, qkv, stride, layer_kv, (int)n, (int)nh, (int)nkv, max_seq, win, out);

@@ -90,6 +90,43 @@ def test_runner_sliding_window_matches_oracle(gpu, heads, kv_heads, window, n, m
     assert outs[0] == outs[1]
 
 
+@pytest.mark.parametrize("heads,kv_heads,window,n,max_seq", [(64, 8, 12, 700, 768), (32, 32, 40, 650, 700)])
+def test_sliding_window_on_a_long_prompt(gpu, heads, kv_heads, window, n, max_seq):
+    """Prompts long enough for the fp16-split prefill attention (32-key tiles, two at a time): layer 1's K and V rows,
+    which every row's windowed attention in layer 0 went into, against the oracle's. A score's f32 error is up to 2^-19
+    of Σ|q·k|/√hd in either order of summation. The random model's scores reach the hundred thousands; its key
+    projections are scaled 2^-9 here, queries are formed as keys otherwise are, so 2^9·max|k|²/√hd stands for the
+    largest score and that share of a row bounds its difference."""
+    c = dict(TINY, num_heads=heads, num_kv_heads=kv_heads, max_seq_len=max_seq, sliding_window=window)
+    dts = [Q4_K, Q4_K, Q8_0, Q4_K, Q4_K, Q4_K, Q4_K]
+    m = build_tiny(seed=heads * 7 + window, layer_dtype=dts, c=c)
+    for layer in m["layers"]:
+        d = layer[1].reshape(-1, 144)
+        d[:, :4] = (d[:, :4].copy().view(np.float16) * np.float16(2.0 ** -9)).view(np.uint8)
+    toks = np.random.default_rng(n + window).integers(0, c["vocab_size"], n).astype(np.int32)
+    s, co = O.precompute_rope(max_seq, c["head_dim"], c["rope_base"])
+    kvs = []
+    for w in (window, 0):
+        kv = np.zeros((c["num_layers"], 2, kv_heads, max_seq, c["head_dim"]), np.float32)
+        O.forward_batch(oracle_cfg(dict(c, sliding_window=w)), m["emb"][toks], m["layers"], dts, m["norms"], m["final"],
+                        m["lm"], m["lm_dtype"], s, co, kv)
+        kvs.append(kv)
+    L, r = A.lib(), make_runner(m, c)
+    try:
+        A.check(L.aeth_runner_prefill(r, toks.ctypes.data, n, None, None), "prefill")
+        got, fl = np.empty_like(kvs[0]), ctypes.c_int32()
+        A.check(L.aeth_runner_kv_to_host(r, got.ctypes.data, ctypes.byref(fl)), "kv_to_host")
+    finally:
+        L.aeth_runner_free(r)
+    k0 = kvs[0][0, 0, :, :n].astype(np.float64)
+    tol = 2.0 ** -19 * (2 + 2.0 ** 9 * (k0 * k0).sum(-1).max() / np.sqrt(c["head_dim"]))
+    rows = lambda kv: kv[1, :, :, :n].reshape(-1, c["head_dim"])
+    assert tol < 0.02
+    assert_close_rows(rows(got), rows(kvs[0]), tol=tol, what="layer 1 of the windowed prefill")
+    far = np.abs(rows(kvs[1]) - rows(kvs[0])).max(axis=1) > 10 * tol * np.maximum(1.0, np.abs(rows(kvs[0])).max(axis=1))
+    assert far.mean() > 0.3  # the window matters to many rows
+
+
 def test_window_reaching_past_the_prompt_changes_nothing(gpu):
     """A window at least the sequence length masks no key: logits equal the
     unwindowed runner's bit for bit (prefill and a decode step)."""

@@ -211,6 +211,77 @@ def test_attn_prefill_matches_f64(gpu, n, nh, nkv, max_seq, qs):
     assert np.abs(got - ref).max() < 1e-5
 
 
+def attn_prefill64(q, kv, n, nh, nkv, hd):
+    """Causal attention in float64, and per output the sum of |p·v| (the scale of its rounding) and per row the largest
+    Σ|q·k|/√hd of a visible key (the scale of its scores' rounding)."""
+    G, ref, mag, smax = nh // nkv, np.empty((n, nh, hd)), np.empty((n, nh, hd)), np.empty((n, nh, 1))
+    K, V = kv[0].astype(np.float64), kv[1].astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        for h in range(nh):
+            sc = q[:, h * hd:(h + 1) * hd].astype(np.float64) @ K[h // G, :n].T / np.sqrt(hd)
+            sc[np.triu_indices(n, 1)] = -np.inf
+            p = np.exp(sc - sc.max(axis=1, keepdims=True))
+            p /= p.sum(axis=1, keepdims=True)
+            p[np.triu_indices(n, 1)] = 0.0
+            for i in range(n) if not np.isfinite(V[h // G, :n]).all() else ():
+                ref[i, h] = p[i, :i + 1] @ V[h // G, :i + 1]
+            if np.isfinite(V[h // G, :n]).all():
+                ref[:, h] = p @ V[h // G, :n]
+            mag[:, h] = p @ np.abs(V[h // G, :n])
+            a = np.abs(q[:, h * hd:(h + 1) * hd]).astype(np.float64) @ np.abs(K[h // G, :n]).T / np.sqrt(hd)
+            a[np.triu_indices(n, 1)] = 0.0
+            smax[:, h, 0] = a.max(axis=1)
+    return ref, mag, smax
+
+
+# enough rows that the fp16-split kernel takes them (80 pairs of 128/G-query blocks and KV heads): every group size,
+# odd and even block counts, a last key tile of 1 .. 32 keys; key tiles scaled 2^-2 .. 2^2 and value tiles 2^-12 ..
+# 2^12 against each other, so that the tiles' exponents differ
+@pytest.mark.parametrize("n,nh,nkv,max_seq", [(640, 32, 8, 640), (1025, 32, 8, 1100), (700, 64, 8, 704), (1300, 16, 8, 1300),
+                                              (650, 32, 32, 1000)])
+def test_attn_prefill_split_matches_f64(gpu, n, nh, nkv, max_seq):
+    """Error: a score is the f32 sum of 24 matrix-core steps over parts that leave 2^-22 of a product, at most 2^-19 of
+    its Σ|q·k|/√hd = A, which its probability takes on; probabilities and values carry 2^-22 of their own, the sums of
+    at most n/64 + 10 steps less than 2^-19: 2^-19·(2 + A) of Σ|p·v| bounds it."""
+    torch = gpu
+    hd = 128
+    rng = np.random.default_rng(n + nh)
+    stride = (nh + 2 * nkv) * hd
+    q = rng.standard_normal((n, stride)).astype(np.float32)
+    kv = rng.standard_normal((2, nkv, max_seq, hd)).astype(np.float32)
+    for t in range(0, n, 32):
+        kv[0, :, t:t + 32] *= np.float32(2.0) ** rng.integers(-2, 3, (nkv, 1, 1))
+        kv[1, :, t:t + 32] *= np.float32(2.0) ** rng.integers(-12, 13, (nkv, 1, 1))
+    kv[:, :, n:] = np.nan  # slots past the prompt are never read
+    q[5] = 0.0
+    out = torch.empty(n * nh * hd, dtype=torch.float32, device="cuda")
+    qd, kvd = torch.from_numpy(q).cuda(), torch.from_numpy(kv).cuda()
+
+    def run():
+        A.check(A.lib().aeth_attn_prefill(qd.data_ptr(), stride, kvd.data_ptr(), n, nh, nkv, hd, max_seq, out.data_ptr(),
+                                          None), "attn_prefill")
+        torch.cuda.synchronize()
+        return out.cpu().numpy().reshape(n, nh, hd).copy()
+
+    ref, mag, smax = attn_prefill64(q, kv, n, nh, nkv, hd)
+    got = run()
+    assert (np.abs(got - ref) <= 2.0 ** -19 * (2 + smax) * mag).all()
+    assert np.array_equal(run(), got)
+    # one KV head with an infinite key element and an infinite value: its rows as the f32 formula gives them
+    kv[0, 1, n // 2, 3], kv[1, 1, n - 2, 7] = np.inf, -np.inf
+    kvd.copy_(torch.from_numpy(kv))
+    bad, G = run(), nh // nkv
+    mine = np.arange(nh) // G == 1
+    assert np.array_equal(bad[:, ~mine], got[:, ~mine])
+    s = q.reshape(n, -1, hd)[:, :nh][:, mine][n // 2:, :, 3]  # the sign of that key's scores
+    rows = bad[n // 2:, mine]
+    assert np.isnan(rows[s > 0]).all()  # exp(inf - inf)
+    below = np.abs(bad[:n // 2, mine] - ref[:n // 2, mine]) <= 2.0 ** -19 * (2 + smax[:n // 2, mine]) * mag[:n // 2, mine]
+    assert below.all()
+    assert np.isfinite(rows[:n - 2 - n // 2][s[:n - 2 - n // 2] < 0]).all()
+    assert (rows[-2:, :, 7][s[-2:] < 0] == -np.inf).all()
+
+
 # ── device LlamaRunner vs the oracle's decode step ───────────────────────
 
 def make_runner(m, c=TINY):
