@@ -33,6 +33,11 @@
 // the super-block. Per wave: 3 A slots, 2 quant slots, 1 header slot (20 KiB);
 // slice s + 2 is issued before slice s is computed.
 //
+// Up to 32 rows (MT = 1) the second m-tile, which would hold zero rows only, is left
+// out: half the A bytes and MFMAs a slice, and with the LDS that frees one A slot
+// more (slice s + 3). 14336 × 4096 at 7 rows 27.7 → 21.1 µs with prep and split sum
+// (the kernel 19 → 14.6), 4096 × 4096 at 16 rows 23.6 → 18.0.
+//
 // Q5_K (avx2::matmul_q5_k with m rows, src/quant/avx2.rs:97-131) runs the same kernel with a
 // fifth bit per quant: w = d·sc·(q + 16·h) − dmin·m, h bit 32·s + l of the block's qh for
 // element l of sub-block s (q5_k.rs:49-56). q5·sc ≤ 1953 is still an exact fp16 integer, so
@@ -50,37 +55,42 @@
 #include "aeth_gemm_common.hpp"
 #include "aeth_internal.hpp"
 
-#define K8_A 4096   // A fragments of a slice
-#define K8_NA 3     // A slots
 #define K8_W 8      // waves
 
-// LDS of a wave: A slots, the quant slots of a slice pair (Q5_K: + its fifth bits), the
-// header slot of a super-block (Q4_K: + its sub-block sums)
-template <bool Q5>
+// Slots of a wave's ring (MT m-tiles of 32 rows): A fragments of NA slices, the quant slots of two slice pairs
+// (Q5_K: + their fifth bits), the header slot of a super-block (Q4_K: + its sub-block sums). Two m-tiles: 3 A slots,
+// slice s + 2 is issued before slice s is computed; one: 4, slice s + 3.
+template <bool Q5, int MT>
 struct K8L {
+    static constexpr int NA = MT == 2 ? 3 : 4, A = 2048 * MT;
     static constexpr int B = Q5 ? 2560 : 2048;
-    static constexpr int HS = Q5 ? 2048 : 4096;
-    static constexpr int BOFF = K8_NA * K8_A;
+    static constexpr int HS = Q5 ? 2048 : 2048 + 1024 * MT;
+    static constexpr int BOFF = NA * A;
     static constexpr int HOFF = BOFF + 2 * B;
-    static constexpr int WAVE = HOFF + HS;  // 20 KiB (Q4_K), 19 KiB (Q5_K)
+    static constexpr int WAVE = HOFF + HS;  // 20 KiB (Q4_K), 19 KiB (Q5_K) of two m-tiles; 15 KiB of one
 };
 
 // buffer loads issued for slice s (s = position in the wave's run): A fragments, a pair's quants
 // (Q5_K: and fifth bits), a super-block's headers (Q4_K: and sums)
-template <bool Q5>
+template <bool Q5, int MT>
 __host__ __device__ constexpr int k8_loads(int s) {
-    return 4 + ((s & 1) == 0 ? (Q5 ? 4 : 2) : 0) + ((s & 15) == 0 ? (Q5 ? 2 : 4) : 0);
+    return 2 * MT + ((s & 1) == 0 ? (Q5 ? 4 : 2) : 0) + ((s & 15) == 0 ? (Q5 ? 2 : 2 + MT) : 0);
 }
-// loads allowed outstanding when slice position j starts: slice j + 1's, and at j = 0 (Q5_K) the
-// two sub-block-sum loads issued after it, at the end of the previous super-block
-template <bool Q5>
+// loads allowed outstanding when slice position j starts: those of the slices issued after it, and at j = 0
+// (Q5_K) the sub-block-sum loads issued after them, at the end of the previous super-block
+template <bool Q5, int MT>
 __host__ __device__ constexpr int k8_wait(int j) {
-    return k8_loads<Q5>(j + 1) + (Q5 && j == 0 ? 2 : 0);
+    return k8_loads<Q5, MT>(j + 1) + (MT == 1 ? k8_loads<Q5, MT>(j + 2) : 0) + (Q5 && j == 0 ? MT : 0);
+}
+template <int N>
+__device__ __forceinline__ void k8_vm(int n) {  // n is a constant once unrolled
+    if (n == N) vm_wait<N>();
+    else if constexpr (N < 16) k8_vm<N + 1>(n);
 }
 
-template <bool Q5>
+template <bool Q5, int MT>
 __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
-    using L = K8L<Q5>;
+    using L = K8L<Q5, MT>;
     __shared__ __attribute__((aligned(1024))) char smem[K8_W * L::WAVE];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -131,7 +141,7 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
         const int kso = b * 32768 + (4 * J + 2 * nib + kg) * 2048;
         char* st = wl + sa;
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++)
+        for (int mt = 0; mt < MT; mt++)
 #pragma unroll
             for (int p = 0; p < 2; p++)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, (lds_void*)(st + (mt * 2 + p) * 1024), 16, a_v,
@@ -157,7 +167,7 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rH, (lds_void*)(hs + i * 1024), 16, h_v[i], b * 256, 0, 0);
             if constexpr (!Q5) {
 #pragma unroll
-                for (int mt = 0; mt < 2; mt++)
+                for (int mt = 0; mt < MT; mt++)
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rS, (lds_void*)(hs + 2048 + mt * 1024), 16, s_v[mt],
                                                              b * 16, 0, 0);
             }
@@ -166,7 +176,7 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
     // Q5_K: the sub-block sums of super-block b straight into registers
     auto load_sums = [&](int b, half8_t* sv) {
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++)
+        for (int mt = 0; mt < MT; mt++)
             sv[mt] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rS, s_v[mt], b * 16, 0));
     };
 
@@ -176,14 +186,14 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
     // Q5_K: this lane's fifth-bit word of column tile c in a quant slot: + 2048 + 128c
     const int f_off = (lane & 31) * 4 + 2 * (lane >> 5);
 
-    f32x16 U[2][4];
+    f32x16 U[MT][4];
 #pragma unroll
-    for (int mt = 0; mt < 2; mt++)
+    for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int c = 0; c < 4; c++) U[mt][c] = (f32x16){};
     float D[4] = {1.0f, 1.0f, 1.0f, 1.0f};  // current scale of column tile c (this lane's column)
     u32x4 hd[4] = {};
-    half8_t sv[2] = {};
+    half8_t sv[MT] = {};
     half2_t sp[4] = {}, zp[4] = {};
     u32x2 raw[4] = {};
     uint32_t x8[4] = {}, y8[4] = {};
@@ -193,7 +203,8 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
 
     if (ns > 0) {
         issue(sb0, 0, 0);
-        issue(sb0, 1, K8_A);
+        issue(sb0, 1, L::A);
+        if constexpr (MT == 1) issue(sb0, 2, 2 * L::A);
         if constexpr (Q5) load_sums(sb0, sv);
     }
     int s3 = 0;  // (16·bi) mod 3: slice 16·bi + j uses A slot (s3 + j) mod 3
@@ -203,19 +214,19 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
             const int nib = j & 1;
             // slice s has landed when only slice s + 1's loads (and at j = 0 the sums, Q5_K) are
             // outstanding
-            const int nw = k8_wait<Q5>(j);  // 4, 6, 8 or 10 (folded: j is unrolled)
-            if (nw == 10) vm_wait<10>();
-            else if (nw == 8) vm_wait<8>();
-            else if (nw == 6) vm_wait<6>();
-            else vm_wait<4>();
-            {
+            k8_vm<2>(k8_wait<Q5, MT>(j));
+            int sc3;
+            if constexpr (MT == 2) {
                 int sl = s3 + (j + 2) % 3;
                 sl = sl >= 3 ? sl - 3 : sl;
-                issue(sb0 + bi + (j + 2) / 16, (j + 2) & 15, sl * K8_A);
+                issue(sb0 + bi + (j + 2) / 16, (j + 2) & 15, sl * L::A);
+                sc3 = s3 + j % 3;
+                sc3 = sc3 >= 3 ? sc3 - 3 : sc3;
+            } else {  // 16 slices are four rounds of the slots
+                issue(sb0 + bi + (j + 3) / 16, (j + 3) & 15, ((j + 3) & 3) * L::A);
+                sc3 = j & 3;
             }
-            int sc3 = s3 + j % 3;
-            sc3 = sc3 >= 3 ? sc3 - 3 : sc3;
-            const uint32_t sa = wl_lds + sc3 * K8_A;
+            const uint32_t sa = wl_lds + sc3 * L::A;
             const uint32_t sq = wl_lds + L::BOFF + ((j >> 1) & 1) * L::B;
             if (j == 0) {
                 const uint32_t hs = wl_lds + L::HOFF;
@@ -225,7 +236,7 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
                 hd[3] = lds_b128<1536>(hs + h_off);
                 if constexpr (!Q5) {
                     sv[0] = lds_b128h<2048>(hs + a_v);
-                    sv[1] = lds_b128h<3072>(hs + a_v);
+                    if constexpr (MT == 2) sv[MT - 1] = lds_b128h<3072>(hs + a_v);
                 }
             }
             if (nib == 0) {
@@ -243,18 +254,20 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
             if constexpr (Q5) {
                 if (j == 0) lgkm_wait<11>();  // at most 15 LDS reads outstanding: the first header read is back
             }
-            half8_t a[2][2];  // [mt][part]
+            half8_t a[MT][2];  // [mt][part]
             a[0][0] = lds_b128h<0>(sa + a_v);
             a[0][1] = lds_b128h<1024>(sa + a_v);
-            a[1][0] = lds_b128h<2048>(sa + a_v);
-            a[1][1] = lds_b128h<3072>(sa + a_v);
-            lgkm_wait<4>();  // all but the A fragments
+            if constexpr (MT == 2) {
+                a[MT - 1][0] = lds_b128h<2048>(sa + a_v);
+                a[MT - 1][1] = lds_b128h<3072>(sa + a_v);
+            }
+            lgkm_wait<2 * MT>();  // all but the A fragments
             if (j == 0) {
 #pragma unroll
                 for (int c = 0; c < 4; c++) pin(hd[c]);
                 if constexpr (!Q5) {
-                    pin(sv[0]);
-                    pin(sv[1]);
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) pin(sv[mt]);
                 }
                 // entering the super-block: rescale U to this block's d (a zero d keeps the scale;
                 // its weights are zeroed through the scales below)
@@ -265,7 +278,7 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
                     if (bi > 0) {
                         const float r = D[c] * __builtin_amdgcn_rcpf(Dn);  // one rounding per block
 #pragma unroll
-                        for (int mt = 0; mt < 2; mt++)
+                        for (int mt = 0; mt < MT; mt++)
 #pragma unroll
                             for (int q = 0; q < 16; q++) U[mt][c][q] *= r;
                     }
@@ -339,14 +352,14 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
             }
             lgkm_wait<0>();
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++) {
+            for (int mt = 0; mt < MT; mt++) {
                 pin(a[mt][0]);
                 pin(a[mt][1]);
             }
 #pragma unroll
             for (int p = 0; p < 2; p++)
 #pragma unroll
-                for (int mt = 0; mt < 2; mt++)
+                for (int mt = 0; mt < MT; mt++)
 #pragma unroll
                     for (int c = 0; c < 4; c++)
                         U[mt][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][p], bv[c], U[mt][c], 0, 0, 0);
@@ -361,7 +374,7 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
                     bytes_to_h2(((w >> 4) & 0x0F0F0F0Fu) | ((z >> 2) & 0x30303030u), m45, m67);
                     const half8_t mv = {m01[0], m01[1], m23[0], m23[1], m45[0], m45[1], m67[0], m67[1]};
 #pragma unroll
-                    for (int mt = 0; mt < 2; mt++) {
+                    for (int mt = 0; mt < MT; mt++) {
                         const f32x16 q = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv[mt], mv, (f32x16){}, 0, 0, 0);
 #pragma unroll
                         for (int r = 0; r < 16; r++) U[mt][c][r] = fmaf(ndm, q[r], U[mt][c][r]);
@@ -378,47 +391,48 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
     // The eight K-eighth tiles meet in LDS. Round 1: waves 4..7 hand theirs to
     // waves 0..3 (slot [w - 4]); round 2: waves 0..3 write the pair sums and wave w
     // (0..7) sums (mt, c) = (w / 4, w % 4) over them in order and stores it.
-    float* red = (float*)smem;  // [4][2][4][16][64] floats = 128 KiB
+    float* red = (float*)smem;  // [4][MT][4][16][64] floats = 64 KiB a m-tile
     const int mt = wave >> 2, c = wave & 3, lr = lane & 31;
     const int col = n0 + 32 * c + lr;
     int rows[16];
 #pragma unroll
     for (int r = 0; r < 16; r++) rows[r] = m0 + 32 * mt + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
     G2Epi E;  // in flight during the reduction
-    if (nsplit == 1) g2_epi_load(E, G.escale, G.C, G.ldc, G.m, G.n, rows, col, G.accumulate);
+    if (nsplit == 1 && mt < MT) g2_epi_load(E, G.escale, G.C, G.ldc, G.m, G.n, rows, col, G.accumulate);
 #pragma unroll
-    for (int mt = 0; mt < 2; mt++)
+    for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int c = 0; c < 4; c++)
 #pragma unroll
             for (int r = 0; r < 16; r++) U[mt][c][r] *= D[c];
     if (wave >= 4) {
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++)
+        for (int mt = 0; mt < MT; mt++)
 #pragma unroll
             for (int c = 0; c < 4; c++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) red[((((wave - 4) * 2 + mt) * 4 + c) * 16 + r) * 64 + lane] = U[mt][c][r];
+                for (int r = 0; r < 16; r++) red[((((wave - 4) * MT + mt) * 4 + c) * 16 + r) * 64 + lane] = U[mt][c][r];
     }
     __syncthreads();
     if (wave < 4) {
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++)
+        for (int mt = 0; mt < MT; mt++)
 #pragma unroll
             for (int c = 0; c < 4; c++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
-                    const int i = (((wave * 2 + mt) * 4 + c) * 16 + r) * 64 + lane;
+                    const int i = (((wave * MT + mt) * 4 + c) * 16 + r) * 64 + lane;
                     red[i] = U[mt][c][r] + red[i];
                 }
     }
     __syncthreads();
+    if (mt >= MT) return;
     float sum[16];
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-        sum[r] = red[(((0 * 2 + mt) * 4 + c) * 16 + r) * 64 + lane];
+        sum[r] = red[(((0 * MT + mt) * 4 + c) * 16 + r) * 64 + lane];
 #pragma unroll
-        for (int w = 1; w < 4; w++) sum[r] += red[(((w * 2 + mt) * 4 + c) * 16 + r) * 64 + lane];
+        for (int w = 1; w < 4; w++) sum[r] += red[(((w * MT + mt) * 4 + c) * 16 + r) * 64 + lane];
     }
     if (nsplit > 1) {  // the split's partial tile (rows < mp, columns < pld: no bounds to check)
         int ld;
@@ -435,10 +449,12 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
 }
 
 int aeth_gemm_kq_launch(const KqArgs& G, hipStream_t s) {
-    if (G.fifth)
-        hipLaunchKernelGGL(k_gemm_kq<true>, dim3(g2_grid(G)), dim3(64 * K8_W), 0, s, G);
-    else
-        hipLaunchKernelGGL(k_gemm_kq<false>, dim3(g2_grid(G)), dim3(64 * K8_W), 0, s, G);
+    // up to 32 rows: the one-m-tile form (the second m-tile would hold zero rows only)
+    const dim3 grid(g2_grid(G)), block(64 * K8_W);
+    if (G.fifth && G.m <= 32) hipLaunchKernelGGL((k_gemm_kq<true, 1>), grid, block, 0, s, G);
+    else if (G.fifth) hipLaunchKernelGGL((k_gemm_kq<true, 2>), grid, block, 0, s, G);
+    else if (G.m <= 32) hipLaunchKernelGGL((k_gemm_kq<false, 1>), grid, block, 0, s, G);
+    else hipLaunchKernelGGL((k_gemm_kq<false, 2>), grid, block, 0, s, G);
     AETH_LAUNCH_CHECK();
     return g2_split_sum(G, s);
 }

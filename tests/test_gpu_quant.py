@@ -363,6 +363,14 @@ def test_q4k_small_batches(gpu, m, n, k):
     assert_close(got_q8, ref_q8, what="q4_k dot-product mode m=%d n=%d k=%d" % (m, n, k))
 
 
+# Up to 32 rows the Q4_K / Q5_K GEMM leaves out the second m-tile; 33 rows have both. Super-blocks split unevenly over
+# its 8 waves (idle waves at 3 and 4), one and many workgroups along K, ragged n.
+@pytest.mark.parametrize("dtype", [Q4_K, Q5_K])
+@pytest.mark.parametrize("m,n,k", [(17, 130, 768), (31, 40, 2560), (32, 300, 1024), (32, 96, 16384), (33, 48, 1024)])
+def test_gemm_kq_one_m_tile(gpu, dtype, m, n, k):
+    (check_q4k_gemm if dtype == Q4_K else check_q5k_gemm)(gpu, m, n, k)
+
+
 # Small batches of Q8_0 rows (aeth_q80_gemm_rows): the row-batched GEMV until m · (weight bytes)
 # reaches 380 MB for weights up to 32 MiB and 180 MB above (from 3 rows), else the GEMM; both sides
 # of the switch at the measured crossovers, plain, accumulate and the dot-product mode.
