@@ -19,6 +19,7 @@ SOURCES = [
     "aeth_gemv_ext.hip",
     "aeth_gemm.hip",
     "aeth_gemm_kq.hip",
+    "aeth_gemm_q4k_big.hip",
     "aeth_gemm_q6k.hip",
     "aeth_gemm_q80.hip",
     "aeth_gemm_f16.hip",
@@ -46,6 +47,7 @@ def hipcc():
 EXTRA = {
     "aeth_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "aeth_gemm_kq.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "aeth_gemm_q4k_big.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "aeth_gemm_q6k.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "aeth_gemm_q80.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "aeth_gemm_f16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],

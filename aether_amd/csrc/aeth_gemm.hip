@@ -27,8 +27,9 @@
 //
 // This file holds the activation prep (k_gemm_prep), the launcher and the
 // single-K-group kernel for buffers past 32-bit offsets; the default main
-// kernel is the K-split one in aeth_gemm_kq.hip. Both use a workgroup tile of
-// 64 × 128 of C and stage their operands through LDS rings filled with
+// kernel is the K-split one in aeth_gemm_kq.hip, for large products the one on 128 × 256
+// tiles in aeth_gemm_q4k_big.hip. The first two use a workgroup tile of
+// 64 × 128 of C; all stage their operands through LDS rings filled with
 // direct-to-LDS loads (global_load_lds_dwordx4 / buffer_load_dwordx4 … lds: lane
 // i of a wave writes LDS bytes [16i, 16i+16) of the destination, from any
 // address): A as MFMA fragments written by the prep kernel in operand order (so
@@ -666,7 +667,8 @@ int aeth_gemm_q4k_launch(const aeth_weight* w, const float* d_a, int64_t m, floa
                (int)std::min(ab, (int64_t)INT32_MAX), (int)std::min(qb, (int64_t)INT32_MAX),
                (int)std::min(hb, (int64_t)INT32_MAX), d_c, ldc, (flags & AETH_MM_ACCUMULATE) ? 1 : 0, swo ? 1 : 0};
     const bool fits32 = qb < INT32_MAX && ab < INT32_MAX;  // buffer offsets are 32-bit
-    // The K-split kernel (aeth_gemm_kq.hip); the single-K-group kernel serves buffers past the 32-bit
+    // The K-split kernel (aeth_gemm_kq.hip), for Q4_K products of enough 128 × 256 tiles the one that shares operands
+    // through LDS (aeth_gemm_q4k_big.hip: K whole in each workgroup, no partial tiles); the single-K-group kernel serves buffers past the 32-bit
     // offsets of the buffer loads, and AETH_GEMM_KERNEL=2 forces it (tests)
     static const int env_kernel = getenv("AETH_GEMM_KERNEL") ? atoi(getenv("AETH_GEMM_KERNEL")) : 0;
     if (fits32 && (env_kernel != 2 || q5)) {
@@ -674,12 +676,13 @@ int aeth_gemm_q4k_launch(const aeth_weight* w, const float* d_a, int64_t m, floa
         // round of workgroups (each wave keeps at least one super-block), the partial tiles in the
         // stream's scratch (not with a caller's workspace)
         SplitPlan P;
-        if ((rc = split_plan(s, gm, gn, nb / 8, ws != nullptr, P))) return rc;
+        const bool big = !q5 && aeth_q4k_big_ok(m, w->n);
+        if ((rc = split_plan(s, gm, gn, nb / 8, ws != nullptr || big, P))) return rc;
         KqArgs Q{(const uint8_t*)frag, (const uint8_t*)Sh, esc, w->p0, w->p1, (int)m, (int)w->n, k, nb, (int)ntiles,
                  (int)mp, gm, gn, (int)ab, (int)(mp * (k / 32) * 4), (int)qb, (int)std::min(hb, (int64_t)INT32_MAX),
                  d_c, ldc, (flags & AETH_MM_ACCUMULATE) ? 1 : 0, swo ? 1 : 0, P.ksplit, P.part, gn * G2_BN,
                  q5 ? w->p3 : nullptr, q5 ? (int)(ntiles * nb * 512) : 0, P.t_full, P.tsplit};
-        return aeth_gemm_kq_launch(Q, s);
+        return big ? aeth_gemm_q4k_big_launch(Q, s) : aeth_gemm_kq_launch(Q, s);
     }
     hipLaunchKernelGGL(k_gemm_q4k_ring, dim3((unsigned)(gm * gn)), dim3(256), 0, s, G);
     AETH_LAUNCH_CHECK();

@@ -233,6 +233,9 @@ struct KqArgs {
     int t_full = 0, tsplit = 1;
 };
 int aeth_gemm_kq_launch(const KqArgs& G, hipStream_t s);
+// The Q4_K GEMM on 128 × 256 workgroup tiles (aeth_gemm_q4k_big.hip), and whether m × n outputs are enough of them
+bool aeth_q4k_big_ok(int64_t m, int64_t n);
+int aeth_gemm_q4k_big_launch(KqArgs G, hipStream_t s);
 
 // The second kernel of a GEMM split over K across workgroups (aeth_gemm_q6k.hip): the splits'
 // tile sums part[split][row][col] (rows mp, pld columns) added in split order, then the

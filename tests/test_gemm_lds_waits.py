@@ -29,7 +29,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "aether_amd", "csrc")
 # the kernels with inline-asm LDS reads, and aeth_gemm.hip's compiler-scheduled ones (the checker must pass those)
-SOURCES = ["aeth_gemm_kq.hip", "aeth_gemm_q6k.hip", "aeth_gemm_q80.hip", "aeth_gemm.hip", "aeth_prefill.hip"]
+SOURCES = ["aeth_gemm_kq.hip", "aeth_gemm_q4k_big.hip", "aeth_gemm_q6k.hip", "aeth_gemm_q80.hip", "aeth_gemm.hip", "aeth_prefill.hip"]
 
 _REG_RANGE = re.compile(r"\b([va])\[(\d+):(\d+)\]")
 _REG_ONE = re.compile(r"\b([va])(\d+)\b")

@@ -371,6 +371,30 @@ def test_gemm_kq_one_m_tile(gpu, dtype, m, n, k):
     (check_q4k_gemm if dtype == Q4_K else check_q5k_gemm)(gpu, m, n, k)
 
 
+# The Q4_K GEMM of 128 × 256 workgroup tiles (aeth_q4k_big_ok: enough of them to fill the CUs): a last m-tile pair
+# past the 64-row tiles of A (530), ragged last rows and columns, one super-block, more columns than tiles of 16.
+@pytest.mark.parametrize("m,n,k", [(512, 12288, 256), (530, 11000, 768), (100, 49140, 256), (449, 12300, 512)])
+def test_gemm_q4k_big_tiles(gpu, m, n, k):
+    """Per-row exponents, accumulate (check_q4k_gemm's bars), and the plain rows against the f64 product: A's split
+    leaves 2^-22 of a product, the sum runs through 32 MFMAs of 8 products each a super-block (4 roundings each, hi and
+    lo), then one fused add per super-block for the scales and one for the mins."""
+    check_q4k_gemm(gpu, m, n, k)
+    rng = np.random.default_rng(m + n + k)
+    raw = weight(Q4_K, n, k, 5 * n + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    w = make_weight(gpu, Q4_K, n, k, raw)
+    got = gemv(gpu, w, x.ravel(), n, m)
+    A.lib().aeth_weight_free(w)
+    # |w| <= 945·d + 63·dmin before the offsets cancel: bound the terms by both parts' magnitudes
+    w64 = O.dequant(Q4_K, raw, n * k).reshape(n, k).astype(np.float64)
+    blk = raw.reshape(-1, 144)
+    dmin = np.array([abs(float(O.decode_d(int(v)))) for v in blk[:, 2:4].copy().view(np.uint16)[:, 0]])
+    off = np.repeat(63.0 * dmin, 256).reshape(n, k)
+    x64 = x.astype(np.float64)
+    bound = (32 * 4 * 2 + 2 * (k // 256) + 8) * 2.0 ** -24 * (np.abs(x64) @ (np.abs(w64) + 2 * off).T)
+    assert (np.abs(got - x64 @ w64.T) <= bound).all()
+
+
 # Small batches of Q8_0 rows (aeth_q80_gemm_rows): the row-batched GEMV until m · (weight bytes)
 # reaches 380 MB for weights up to 32 MiB and 180 MB above (from 3 rows), else the GEMM; both sides
 # of the switch at the measured crossovers, plain, accumulate and the dot-product mode.
