@@ -618,6 +618,20 @@ int aeth_embed_launch(const float* table, const int* d_token, int64_t token, int
     return AETH_OK;
 }
 
+// Sets the device decode state {token, pos, fill, next token, generate step}: from the
+// launch's arguments, where a copy from host memory would be waited for.
+__global__ void k_state_set(int* st, int token, int pos, int fill) {
+    const int v[5] = {token, pos, fill, token, 0};
+    if (threadIdx.x == 0)
+        for (int i = 0; i < 5; i++) st[i] = v[i];
+}
+
+int aeth_state_set_launch(int* st, int token, int pos, int fill, hipStream_t s) {
+    hipLaunchKernelGGL(k_state_set, dim3(1), dim3(64), 0, s, st, token, pos, fill);
+    AETH_LAUNCH_CHECK();
+    return AETH_OK;
+}
+
 // Advances the device decode state {token, pos, fill} after a step:
 // StaticKVCache::advance (kv_cache.rs:67-71) and pos += 1; the next token was
 // written by the argmax.

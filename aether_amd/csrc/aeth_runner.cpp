@@ -50,6 +50,7 @@ struct aeth_runner {
     unsigned long long* amax = nullptr;  // fused LM-head argmax key (reset by the state kernel)
     int* tok_out = nullptr;  // [max_seq] greedy tokens of the current generate call, by step
     int fill = 0;           // host mirror of the cache fill
+    uint8_t* host_out = nullptr;  // pinned: a step's next token (16 bytes), then its logits
     hipGraphExec_t graph = nullptr;
     // batched prefill buffers (grow-only): rows of x, normed x, q|k|v, attention
     // output, interleaved gate|up, SiLU product; prompt token ids
@@ -64,6 +65,8 @@ struct aeth_runner {
 };
 
 namespace {
+
+constexpr size_t HOST_TOK = 16;  // aeth_runner::host_out: bytes before the logits
 
 const int64_t kKvd(const aeth_llama_config& c) { return (int64_t)c.num_kv_heads * c.head_dim; }
 
@@ -169,6 +172,7 @@ void runner_release(aeth_runner* r) {
                     r->p_x, r->p_n, r->p_qkv, r->p_att, r->p_gu, r->p_h, r->p_tok};
     for (void* b : bufs)
         if (b) hipFree(b);
+    if (r->host_out) hipHostFree(r->host_out);
     if (r->stream) {
         aeth_stream_scratch_release(r->stream);  // the GEMM / GGUF-order scratch of this runner's stream
         hipStreamDestroy(r->stream);
@@ -261,6 +265,7 @@ int enqueue_step(aeth_runner* r) {
 }
 
 int set_state(aeth_runner* r, int token, int pos);
+int step_results(aeth_runner* r, float* logits, int32_t* next_token);
 
 // Batched prefill (forward_batch, runner.rs:833-993; LlamaRunner::prefill :695-704):
 // tokens at positions 0..n-1, K/V at cache slots 0..n-1, per layer
@@ -396,19 +401,33 @@ int runner_prefill_locked(aeth_runner* r, const int32_t* tokens, int32_t n, floa
     r->fill = n - 1;
     if ((rc = set_state(r, tokens[n - 1], n - 1))) return rc;
     if ((rc = enqueue_head(r))) return rc;
-    if (logits)
-        AETH_HIP_CHECK(hipMemcpyAsync(logits, r->logits, sizeof(float) * c.vocab_size, hipMemcpyDeviceToHost, s));
-    int tok = 0;
-    AETH_HIP_CHECK(hipMemcpyAsync(&tok, r->st + 3, sizeof(int), hipMemcpyDeviceToHost, s));
-    AETH_HIP_CHECK(hipStreamSynchronize(s));
+    if ((rc = step_results(r, logits, next_token))) return rc;
     r->fill = n;
-    if (next_token) *next_token = tok;
     return AETH_OK;
 }
 
-int set_state(aeth_runner* r, int token, int pos) {
-    int h[5] = {token, pos, r->fill, token, 0};  // + the generate step counter
-    AETH_HIP_CHECK(hipMemcpyAsync(r->st, h, sizeof(h), hipMemcpyHostToDevice, r->stream));
+int set_state(aeth_runner* r, int token, int pos) { return aeth_state_set_launch(r->st, token, pos, r->fill, r->stream); }
+
+// Waits for the step and hands out what the caller asked for (either may be NULL). Through the runner's pinned
+// buffer: a copy to pageable memory is staged by the driver in pieces it waits for (a 200-token prefill and six
+// steps of a 4-layer 8B-wide model, 32000 logits each: 3288 → 3079 µs). Memory that the driver knows
+// (pinned by the caller) is the copy's target itself.
+int step_results(aeth_runner* r, float* logits, int32_t* next_token) {
+    const size_t lb = sizeof(float) * (size_t)r->cfg.vocab_size;
+    bool staged = r->host_out != nullptr;
+    if (staged && logits) {
+        hipPointerAttribute_t at;
+        if (hipPointerGetAttributes(&at, logits) != hipSuccess) (void)hipGetLastError();
+        else staged = at.type == hipMemoryTypeUnregistered;
+    }
+    int tok = 0;
+    float* const ldst = staged ? (float*)(r->host_out + HOST_TOK) : logits;
+    int* const tdst = r->host_out ? (int*)r->host_out : &tok;
+    if (logits) AETH_HIP_CHECK(hipMemcpyAsync(ldst, r->logits, lb, hipMemcpyDeviceToHost, r->stream));
+    if (next_token) AETH_HIP_CHECK(hipMemcpyAsync(tdst, r->st + 3, sizeof(int), hipMemcpyDeviceToHost, r->stream));
+    AETH_HIP_CHECK(hipStreamSynchronize(r->stream));
+    if (logits && staged) memcpy(logits, ldst, lb);
+    if (next_token) *next_token = *tdst;
     return AETH_OK;
 }
 
@@ -572,6 +591,10 @@ int runner_create_impl(const aeth_llama_config* cfg, const void* const* layer_we
     RC(dmalloc((uint8_t**)&r->am_ws, aeth_argmax_ws_bytes()));
     RC(dmalloc(&r->st, 5));
     RC(dmalloc(&r->tok_out, c.max_seq_len));
+    if (hipHostMalloc((void**)&r->host_out, HOST_TOK + sizeof(float) * (size_t)c.vocab_size, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        r->host_out = nullptr;  // the results are then copied to the caller's memory directly
+    }
     if (hipStreamSynchronize(s) != hipSuccess) {
         return aeth_set_error(AETH_EHIP, "runner: setup sync failed");
     }
@@ -650,14 +673,8 @@ static int runner_decode_locked(aeth_runner* r, int32_t token, int32_t pos, floa
     r->partial_valid = false;
     if ((rc = set_state(r, token, pos))) return rc;
     if ((rc = enqueue_step(r))) return rc;
-    if (logits)
-        AETH_HIP_CHECK(hipMemcpyAsync(logits, r->logits, sizeof(float) * r->cfg.vocab_size, hipMemcpyDeviceToHost,
-                                      r->stream));
-    int tok = 0;
-    AETH_HIP_CHECK(hipMemcpyAsync(&tok, r->st + 3, sizeof(int), hipMemcpyDeviceToHost, r->stream));
-    AETH_HIP_CHECK(hipStreamSynchronize(r->stream));
+    if ((rc = step_results(r, logits, next_token))) return rc;
     if (r->fill < r->cfg.max_seq_len) r->fill++;
-    if (next_token) *next_token = tok;
     return AETH_OK;
 }
 
@@ -910,10 +927,7 @@ extern "C" AETHER_API int aether_decode_budgeted(aether_model* m, int token, int
     }
     r->partial_valid = false;
     if (enqueue_head(r)) return AETHER_ERR;
-    if (hipMemcpyAsync(logits_out, r->logits, sizeof(float) * r->cfg.vocab_size, hipMemcpyDeviceToHost, r->stream) !=
-            hipSuccess ||
-        hipStreamSynchronize(r->stream) != hipSuccess)
-        return AETHER_ERR;
+    if (step_results(r, logits_out, nullptr)) return AETHER_ERR;
     if (r->fill < r->cfg.max_seq_len) r->fill++;
     return AETHER_OK;
 }

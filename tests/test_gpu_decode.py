@@ -489,6 +489,41 @@ def test_runner_gguf_order_formats(gpu, mix, lm_dtype):
     assert outs[0] == outs[1]
 
 
+# The step's results reach pageable memory through the runner's pinned buffer and pinned memory directly;
+# either output may be NULL. The same prompt and step give the same bytes each way.
+@pytest.mark.parametrize("vocab", [3, 512, 1283])
+def test_runner_results_by_destination(gpu, vocab):
+    c = dict(TINY, vocab_size=vocab)
+    m = build_tiny(seed=23, c=c)
+    r = make_runner(m, c)
+    L = A.lib()
+    toks = (np.arange(9) % vocab).astype(np.int32)
+    pinned = gpu.empty(vocab, pin_memory=True)
+    pageable = np.empty(vocab + 1, dtype=np.float32)
+    nxt = ctypes.c_int32()
+    try:
+        def turn(dst, token):
+            got = []
+            for call in (lambda p, t: L.aeth_runner_prefill(r, toks.ctypes.data, len(toks), p, t),
+                         lambda p, t: L.aeth_runner_decode(r, vocab - 1, len(toks), p, t)):
+                pinned.fill_(-7.0)
+                pageable.fill(-7.0)
+                nxt.value = -1
+                A.check(call(None if dst is None else dst.ctypes.data if dst is pageable else dst.data_ptr(),
+                             ctypes.byref(nxt) if token else None), "step")
+                assert pageable[vocab] == -7.0
+                got.append((np.asarray(dst[:vocab]).copy() if dst is not None else None, nxt.value if token else None))
+            return got
+
+        want = turn(pinned, True)
+        for dst, token in ((pageable, True), (pageable, False), (pinned, False), (None, True), (None, False)):
+            for (a, t), (b, u) in zip(want, turn(dst, token)):
+                assert b is None or np.array_equal(a, b)
+                assert u is None or u == t == O.argmax(a)
+    finally:
+        L.aeth_runner_free(r)
+
+
 def test_runner_prefill_bad_arguments(gpu):
     m = build_tiny(seed=8)
     r = make_runner(m)
