@@ -4,10 +4,12 @@
 // "Exact" mode on fp16 MFMA (v_mfma_f32_32x32x16_f16, fp32 accumulate):
 //  * A is split into two fp16 parts, A·2^-e = Ah + Al (Ah = fp16(A·2^-e),
 //    Al = fp16(A·2^-e − Ah)): 22 significant bits, f32-level. The power of two
-//    2^e is chosen per row so that its largest value lies in [2^13, 2^14): the
-//    parts stay in fp16 range, and the lo parts of what matters to the row out of
-//    its subnormals (a row of 1e-4 unscaled keeps 13 bits; a shared exponent for
-//    several rows would do the same to a small row next to a large one).
+//    2^e is chosen per row: 0 while its largest value lies in [2^-3, 2^14), otherwise
+//    such that it lies in [2^13, 2^14): the parts stay in fp16 range, and the lo parts
+//    of what matters to the row out of its subnormals (a row of 1e-4 unscaled keeps 13
+//    bits; a shared exponent for several rows would do the same to a small row next to
+//    a large one). Rows that need no scale get none: with every row scaled up the lo parts
+//    carry more set bits into the matrix cores, and the GEMMs took 0.3 .. 0.5 % longer.
 //  * Q4_K weights become exact fp16 integers w = q·sc (q ≤ 15, sc ≤ 63), so
 //    every MFMA product is exact and the K-sum is an f32 accumulation.
 //  * Per 256-element super-block b:  C += 2^e·(d_b·Σ A·(q·sc) − dmin_b·Σ_s m_s·S_s)
@@ -58,7 +60,10 @@
 #define G2_LOADS 6
 
 // ── activation prep (f32 A [m][k]; rows m..mp-1 read as zero). Writes
-//  * escale[r] = 2^e, e the least (from −100 on) with |A[r]·2^-e| < 2^14;
+//  * escale[r] = 2^e, e = 0 if 2^-3 <= max |A[r]| < 2^14, else the least (from −100 on)
+//    with |A[r]·2^-e| < 2^14 (INF, the F16 product's: always that, as its weights are no
+//    integers, and an infinite element gives hi = ±Inf, lo = 0 and is left out of the maximum;
+//    as a test of every element at run time that cost the other GEMMs 1.5 % of their time);
 //  * fragment (mt, ks, part) = 1 KiB at ((mt·nks + ks)·2 + part)·1024 bytes
 //    (nks = k/16): lane l holds row 32·mt + l%32 at k-positions
 //    16·ks + 8·(l/32) + perm4(i), i < 8, of A·2^-e, part 0 = hi, 1 = lo;
@@ -100,7 +105,6 @@ struct PrepArgs {
     int m, k;
     float* escale;
     _Float16 *frag, *Sh, *Sl;
-    int keep_inf;         // an infinite element: hi = ±Inf, lo = 0, the row's scale from its finite ones (F16 weights)
 };
 
 // 8 consecutive floats at p (16-byte aligned when AL16)
@@ -119,7 +123,7 @@ __device__ __forceinline__ void prep_ld8(const float* __restrict__ p, float* v) 
 // SPW: steps a wave holds in registers, at least its share ⌈S/4⌉ (1, 2, 4 or 8: k ≤ 16384 in one chunk).
 // PREP_ROWS: rows per workgroup, 4 (2 where the producer's 8 steps of inputs need more than the
 // 128 registers of a 16-wave workgroup; 1 for at most 128 rows, which then take more CUs).
-template <bool AL16, bool Q8, int MODE, int SPW, int PREP_ROWS>
+template <bool AL16, bool Q8, int MODE, int SPW, int PREP_ROWS, bool INF>
 __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs P) {
     static_assert(!Q8 || MODE == PREP_PLAIN, "the producers feed the exact mode");
     constexpr int WK = PREP_WK;
@@ -202,7 +206,7 @@ __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 const float av = fabsf(v[t][i]);
-                mx = fmaxf(mx, P.keep_inf && av == INFINITY ? 0.0f : av);
+                mx = fmaxf(mx, INF && av == INFINITY ? 0.0f : av);
             }
     }
     mx = aeth_wave_max(mx);
@@ -213,7 +217,7 @@ __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs
     for (int q = 0; q < WK; q++) mx = fmaxf(mx, red[1][PREP_ROWS * q + ri]);
     int E = 14;
     if (mx > 0.0f && isfinite(mx)) (void)frexpf(mx, &E);
-    const float esc = ldexpf(1.0f, max(E - 14, -100));
+    const float esc = ldexpf(1.0f, INF || E > 14 || E < -2 ? max(E - 14, -100) : 0);
     if (j == 0 && lane == 0) P.escale[r] = esc;
     const float inv = 1.0f / esc;  // a power of two: the products below are exact scalings
     const int tp = tid % (64 * PREP_ROWS);  // thread of the part's PREP_ROWS waves
@@ -258,7 +262,7 @@ __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs
                 const float tv = x[perm4(i)] * inv;
                 const _Float16 th = (_Float16)tv;
                 hi[i] = th;
-                lo[i] = P.keep_inf && fabsf(tv) == INFINITY ? (_Float16)0.0f : (_Float16)(tv - (float)th);
+                lo[i] = INF && fabsf(tv) == INFINITY ? (_Float16)0.0f : (_Float16)(tv - (float)th);
             }
             if (sl && gi < ng && (lane & 3) == 0) {  // gi < ng is uniform per four lanes (ng % 32 == 0)
                 const float sv = sum * inv * 0.03125f;
@@ -499,20 +503,20 @@ int64_t aeth_gemm_ws_bytes(int64_t m, int64_t k) {
     return mp * k * 2 * 2 + mp * (k / 32) * 2 * 2 + mp * 4 + 256;
 }
 
-template <bool AL16, bool Q8, int MODE, int SPW>
+template <bool AL16, bool Q8, int MODE, int SPW, bool INF>
 static void prep_launch_r(unsigned mp, hipStream_t s, const PrepArgs& P) {
     constexpr int R = SPW == 8 && MODE != PREP_PLAIN ? 2 : 4;
     if (mp <= 128)  // few rows: one row per workgroup, so that they spread over more CUs
-        hipLaunchKernelGGL((k_gemm_prep<AL16, Q8, MODE, SPW, 1>), dim3(mp), dim3(64 * PREP_WK), 0, s, P);
+        hipLaunchKernelGGL((k_gemm_prep<AL16, Q8, MODE, SPW, 1, INF>), dim3(mp), dim3(64 * PREP_WK), 0, s, P);
     else
-        hipLaunchKernelGGL((k_gemm_prep<AL16, Q8, MODE, SPW, R>), dim3(mp / R), dim3(64 * R * PREP_WK), 0, s, P);
+        hipLaunchKernelGGL((k_gemm_prep<AL16, Q8, MODE, SPW, R, INF>), dim3(mp / R), dim3(64 * R * PREP_WK), 0, s, P);
 }
-template <bool AL16, bool Q8, int MODE>
+template <bool AL16, bool Q8, int MODE, bool INF = false>
 static void prep_launch(int spw, unsigned mp, hipStream_t s, const PrepArgs& P) {
-    if (spw == 1) prep_launch_r<AL16, Q8, MODE, 1>(mp, s, P);
-    else if (spw == 2) prep_launch_r<AL16, Q8, MODE, 2>(mp, s, P);
-    else if (spw == 4) prep_launch_r<AL16, Q8, MODE, 4>(mp, s, P);
-    else prep_launch_r<AL16, Q8, MODE, 8>(mp, s, P);
+    if (spw == 1) prep_launch_r<AL16, Q8, MODE, 1, INF>(mp, s, P);
+    else if (spw == 2) prep_launch_r<AL16, Q8, MODE, 2, INF>(mp, s, P);
+    else if (spw == 4) prep_launch_r<AL16, Q8, MODE, 4, INF>(mp, s, P);
+    else prep_launch_r<AL16, Q8, MODE, 8, INF>(mp, s, P);
 }
 
 // The activation prep of the Q4_K and Q6_K GEMMs: A (or, with `in`, its producer's input) into
@@ -539,9 +543,11 @@ static int gemm_prep(const float* d_a, int64_t m, int k, unsigned flags, const G
     // registers per wave: its share of the row's steps, rounded up to 1, 2, 4 or 8 (past 8: chunks)
     const int share = (int)aeth_cdiv(aeth_cdiv(k, 512), PREP_WK);
     const int spw = share <= 1 ? 1 : share <= 2 ? 2 : share <= 4 ? 4 : 8;
-    const PrepArgs P{d_a, in ? in->norm_w : nullptr, in ? in->eps : 0.0f, (int)m, k, esc, frag, Sh, Sl, keep_inf ? 1 : 0};
+    const PrepArgs P{d_a, in ? in->norm_w : nullptr, in ? in->eps : 0.0f, (int)m, k, esc, frag, Sh, Sl};
     const unsigned pg = (unsigned)mp;  // fragment rows (whole 64-row tiles)
-    if (mode == PREP_RMSNORM) prep_launch<true, false, PREP_RMSNORM>(spw, pg, s, P);
+    if (keep_inf && al16) prep_launch<true, false, PREP_PLAIN, true>(spw, pg, s, P);
+    else if (keep_inf) prep_launch<false, false, PREP_PLAIN, true>(spw, pg, s, P);
+    else if (mode == PREP_RMSNORM) prep_launch<true, false, PREP_RMSNORM>(spw, pg, s, P);
     else if (mode == PREP_SWIGLU) prep_launch<true, false, PREP_SWIGLU>(spw, pg, s, P);
     else if (al16 && q8) prep_launch<true, true, PREP_PLAIN>(spw, pg, s, P);
     else if (q8) prep_launch<false, true, PREP_PLAIN>(spw, pg, s, P);

@@ -371,6 +371,33 @@ def test_gemm_kq_one_m_tile(gpu, dtype, m, n, k):
     (check_q4k_gemm if dtype == Q4_K else check_q5k_gemm)(gpu, m, n, k)
 
 
+@pytest.mark.parametrize("dtype", [Q4_K, Q5_K, Q6_K, Q8_0])
+def test_gemm_row_exponents(gpu, dtype):
+    """Rows from 2^-60 to 2^20 through the activation split of the exact-mode GEMMs, on both sides of the magnitudes where
+    a row takes a power of two (2^-3, 2^14). The parts leave 2^-22 of a value and 2^-22 of the row's largest; the sum
+    runs through 2·k/8 products a wave and a tree; terms are bounded with the two parts of a weight that cancel."""
+    m, n, k = 64, 1024, 4096
+    rng = np.random.default_rng(dtype)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    for i, e in enumerate((-60, -24, -13, -4, -3, -2, -1, 0, 13, 14, 20)):  # max |x[i]| = 0.75·2^e
+        x[i] *= np.float32(0.75 * 2.0 ** e) / np.abs(x[i]).max()
+    raw = weight(dtype, n, k, 3 + dtype)
+    w = make_weight(gpu, dtype, n, k, raw)
+    got = gemv(gpu, w, x, n, m)
+    A.lib().aeth_weight_free(w)
+    x64, w64 = x.astype(np.float64), O.dequant(dtype, raw, n * k).reshape(n, k).astype(np.float64)
+    off = np.zeros((n, k))
+    if dtype in (Q4_K, Q5_K):
+        dmin = raw.reshape(-1, GEOM[dtype][1])[:, 2:4].copy().view(np.float16)[:, 0].astype(np.float64)
+        off = np.repeat(63.0 * dmin, 256).reshape(n, k)
+    wm = np.abs(w64) + 2 * off
+    bound = (2 * k / 64 + 40) * 2.0 ** -24 * (np.abs(x64) @ wm.T) + \
+        2.0 ** -22 * np.abs(x64).max(axis=1, keepdims=True) * wm.sum(axis=1)
+    assert (np.abs(got - x64 @ w64.T) <= bound).all()
+    ref = x64 @ w64.T  # and no row has more than 2e-6 of its own size as its error (a row of 2^-24 without a scale: 1e-1)
+    assert (np.linalg.norm(got - ref, axis=1) <= 2e-6 * np.linalg.norm(ref, axis=1)).all()
+
+
 # The Q4_K GEMM of 128 × 256 workgroup tiles (aeth_q4k_big_ok: enough of them to fill the CUs): a last m-tile pair
 # past the 64-row tiles of A (530), ragged last rows and columns, one super-block, more columns than tiles of 16.
 @pytest.mark.parametrize("m,n,k", [(512, 12288, 256), (530, 11000, 768), (100, 49140, 256), (449, 12300, 512)])
