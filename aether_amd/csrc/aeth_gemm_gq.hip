@@ -5,11 +5,15 @@
 // d (and dmin) per 256 outputs and W[i][j] = d_i·v_ij (Q3_K, v = (sc − 32)·(q − 4)) or d_i·v_ij − dmin_i·m_ij
 // (Q2_K, v = sc·q, m the 4-bit min of j's 16 outputs), where v and m are small integers:
 //   C[r][j] = Σ_i (A[r][i]·d_i)·v_ij − Σ_i (A[r][i]·dmin_i)·m_ij.
-// Per (row, 256 outputs) x_i = A[r][i]·d_i becomes an integer of 31 bits against the largest |x_i| of the row —
-// formed from the product and its rounding error, so the conversion truncates once, below 2^-29 of that
-// maximum — and four balanced signed byte digits of it are four A operands of v_mfma_i32_32x32x32_i8. The i32
+// Per (row, 256 outputs, K part) x_i = A[r][i]·d_i becomes an integer of 31 bits against the largest |x_i| of
+// those inputs — formed from the product and its rounding error, so the conversion truncates once, below 2^-29 of
+// that maximum — and four balanced signed byte digits of it are four A operands of v_mfma_i32_32x32x32_i8. The i32
 // sums are exact (2^14·k), the digits meet in f64 and one rounding to f32 is left: 2.5e-8 of a result, what the
-// f64 product (a dequantized weight and rocBLAS DGEMM) gave before.
+// f64 product (a dequantized weight and rocBLAS DGEMM) gave before. 31 bits do as long as the maximum is not far above
+// the rest, an activation or a block scale out of proportion, whose integer weight may well be 0 in an output: a unit
+// is to stay below 2^-24 of the geometric mean of the sums of four |x_i|, that is, the maximum below 2^5 of it (normal
+// activations under half-normal scales reach 2^2.5, behind a SiLU gate 2^4). Where some row of a workgroup has more, it
+// takes a second product, of the next 30 bits (one run, Q3_K 203 × 4096 × 4096: 49.5 µs without, 75 .. 82 with).
 //
 //  1. k_gq_prep: the blocks unpacked to v (int8) in MFMA operand order, and d as f32.
 //  2. k_gq_gemm: workgroup = 64 rows × 256 outputs. A first pass over its A finds each row's largest |A·d|; then
@@ -17,12 +21,12 @@
 //     rows by 64 outputs, 16 MFMAs between two barriers; of the two waves of a SIMD one converts the next
 //     64 inputs while the other multiplies. When the tiles are few, K is split over workgroups and the f64
 //     partial results (scaled by their own exponents) are added in order (k_narrow).
-// A row of whose products one is not finite (an infinite or NaN activation, or an overflow) is summed in
-// f64 element by element instead, as the f64 product did.
+// A row of whose products one is not finite (an infinite or NaN activation, or an overflow), or of which 61 bits would
+// not do, is summed in f64 element by element instead, as the f64 product did.
 //
 // What bounds it: bytes into the CUs (per 64 inputs 16 KiB of A and twice 16 KiB of v for 1024 clocks of MFMA;
 // without the products the kernel still takes three quarters of its time), then the first pass over A. Q3_K, m =
-// 203, 4096 × 4096: 197 → 48.8 µs (unpack 9.3, product 33, sum 6.3), m = 512, 14336 × 4096: 1197 → 206 µs.
+// 203, 4096 × 4096: 189 → 45 µs (unpack 9.3, product 33, sum 6.3), m = 512, 14336 × 4096: 1197 → 196 µs.
 #include <math.h>
 #include <stdint.h>
 
@@ -38,7 +42,9 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
 #define GQ_KS 64        // inputs per step
-#define GQ_BAD 0x7FFF   // exponent of a row with a product that is not finite
+#define GQ_BAD 0x7FFF   // exponent of a row that is summed element by element
+#define GQ_NAN 0x7FFE   // exponent of a row with a NaN activation: its outputs are NaN
+#define GQ_LOW 30       // bits of the second product
 
 struct GqArgs {
     const uint8_t* raw;   // [k][n/256] blocks
@@ -49,7 +55,7 @@ struct GqArgs {
     int8_t* mins;         // Q2_K: [nB][kp/32][64 lanes][16], 16 columns of 32 used
     float* dmin;
     int gm, ksplit;
-    double* part;         // ksplit > 1: [ksplit][m][n]
+    double* part;         // [ksplit][m][n]: the parts' results, or those of a first product
     float* C;
     int64_t ldc;
     int accumulate;
@@ -181,47 +187,55 @@ __device__ __forceinline__ int gq_trunc(float f) {  // the instruction's own rul
     return i;
 }
 
-template <int F, bool AL16>
-__global__ void __launch_bounds__(512) k_gq_gemm(GqArgs G) {
-    constexpr bool MIN = Gq<F>::MIN;
+// a·d's integer part as bytes of four digits, 0 .. 2 biased by 128; LOW: the GQ_LOW bits behind it
+template <bool LOW> __device__ __forceinline__ uint32_t gq_digits(float a, float d) {
+    const float p = a * d, er = fmaf(a, d, -p);
+    if (!LOW) return (uint32_t)(gq_trunc(p) + gq_trunc(rintf(er))) + 0x808080u;
+    constexpr float up = (float)(1 << GQ_LOW);  // both fractions are exact, their sum is below 1.5
+    return (uint32_t)(gq_trunc((p - truncf(p)) * up) + gq_trunc((er - rintf(er)) * up)) + 0x808080u;
+}
+
+struct GqShared {
     // digit operands [buffer 2][32-input step 2][m-tile 2][digit 4][64 lanes][16 B]: 32 KiB
-    __shared__ __attribute__((aligned(16))) uint8_t dig[2][16384];
-    __shared__ int msum[MIN ? 4 * 64 * 16 : 1];
-    __shared__ int Sx[MIN ? 2 : 1][64];  // the rows' exponents over this workgroup's inputs
-    const int tid = threadIdx.x, lane = tid & 63;
+    uint8_t dig[2][16384];
+    int Sx[2][64];  // the rows' exponents over this workgroup's inputs: of A·d, of A·dmin
+};
+
+// Four floats of A and the scales of a step's inputs, by thread (row tid/8, inputs 4·(tid%8) and 32 on)
+struct GqRaw { float4 a[2], d[2]; };
+template <bool AL16>
+__device__ __forceinline__ void gq_load(const GqArgs& G, const float* a_src, const float* sc, int s, int kq, GqRaw& R) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {  // inputs past k read any value: their d is 0
+        const int i = GQ_KS * s + 32 * j + kq;
+        R.d[j] = *(const float4*)(sc + i);
+        if (AL16) R.a[j] = *(const float4*)(a_src + min(i, G.k - 4));
+        else R.a[j] = make_float4(a_src[min(i, G.k - 1)], a_src[min(i + 1, G.k - 1)], a_src[min(i + 2, G.k - 1)],
+                                  a_src[min(i + 3, G.k - 1)]);
+    }
+}
+
+// The product of one digit set over the steps [s0, s1) of a workgroup. LOW: the second one, added to what the first left
+// in `part`; `more`: a second one follows.
+template <int F, bool AL16, bool LOW>
+__device__ __forceinline__ void gq_product(const GqArgs& G, int tid, int m0, int B, int ks, int s0, int s1, int Srow,
+                                           int Srowm, bool more, GqShared& sh, int* msum) {
+    constexpr bool MIN = Gq<F>::MIN;
+    auto& dig = sh.dig;
+    const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // the XCDs take workgroup ids round robin: each gets a contiguous run of tiles, the row tiles of a block column
-    // next to each other, so that an XCD reads its part of v once
-    const int T = G.gm * G.nB, ks = blockIdx.x / T, id = blockIdx.x - ks * T;
-    const int tile = (T & 7) == 0 ? (id & 7) * (T >> 3) + (id >> 3) : id;
-    const int tm = tile % G.gm, B = tile / G.gm, m0 = 64 * tm;
-    const int nst = G.kp / GQ_KS, s0 = nst * ks / G.ksplit, s1 = nst * (ks + 1) / G.ksplit;
     const int rr = tid >> 3, row = min(m0 + rr, G.m - 1), kq = 4 * (tid & 7);  // this thread's row and inputs of A
     const float* a_src = G.A + (int64_t)row * G.k;
     const float* ds = G.d + (int64_t)B * G.kp;
     const float* dm = G.dmin + (int64_t)B * G.kp;  // MIN only
-
-    struct Raw { float4 a[2], d[2]; };
-    auto loadA = [&](int s, const float* sc, Raw& R) {  // inputs past k read any value: their d is 0
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int i = GQ_KS * s + 32 * j + kq;
-            R.d[j] = *(const float4*)(sc + i);
-            if (AL16) R.a[j] = *(const float4*)(a_src + min(i, G.k - 4));
-            else R.a[j] = make_float4(a_src[min(i, G.k - 1)], a_src[min(i + 1, G.k - 1)], a_src[min(i + 2, G.k - 1)],
-                                      a_src[min(i + 3, G.k - 1)]);
-        }
-    };
-    auto convert = [&](const Raw& R, int S, uint8_t* buf) {
+    auto loadA = [&](int s, const float* sc, GqRaw& R) { gq_load<AL16>(G, a_src, sc, s, kq, R); };
+    auto convert = [&](const GqRaw& R, int S, uint8_t* buf) {
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const float a[4] = {R.a[j].x, R.a[j].y, R.a[j].z, R.a[j].w}, d[4] = {R.d[j].x, R.d[j].y, R.d[j].z, R.d[j].w};
             uint32_t y[4], c[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float as = __builtin_amdgcn_ldexpf(a[e], S), p = as * d[e], er = fmaf(as, d[e], -p);
-                y[e] = (uint32_t)(gq_trunc(p) + gq_trunc(rintf(er))) + 0x808080u;  // bytes: digits 0..2 biased by 128, digit 3
-            }
+            for (int e = 0; e < 4; e++) y[e] = gq_digits<LOW>(__builtin_amdgcn_ldexpf(a[e], S), d[e]);
             gq_transpose(y, c);
             uint32_t* o = (uint32_t*)(buf + j * 8192 + (rr >> 5) * 4096) + ((rr & 31) + 32 * (kq >> 4)) * 4 + ((kq & 15) >> 2);
             o[0] = c[0] ^ 0x80808080u;
@@ -231,47 +245,6 @@ __global__ void __launch_bounds__(512) k_gq_gemm(GqArgs G) {
         }
     };
 
-    int Srow, Srowm = 0;
-    {  // max |A·d| of the row over this workgroup's inputs: the row's eight threads are neighbouring lanes
-        float mx = 0.0f, mxm = 0.0f;
-        bool bad = false;
-        auto most = [&](const float4& a, const float4& d, float& m) {
-            const float x = fmaxf(fmaxf(fabsf(a.x * d.x), fabsf(a.y * d.y)), fmaxf(fabsf(a.z * d.z), fabsf(a.w * d.w)));
-            const float t = fabsf(a.x * d.x) + fabsf(a.y * d.y) + fabsf(a.z * d.z) + fabsf(a.w * d.w);
-            bad |= !(t < INFINITY);  // a NaN or an infinity among them (or four products near overflow)
-            m = fmaxf(m, x);
-        };
-#pragma unroll 4
-        for (int s = s0; s < s1; s++) {
-            Raw R;
-            loadA(s, ds, R);
-            most(R.a[0], R.d[0], mx);
-            most(R.a[1], R.d[1], mx);
-            if constexpr (MIN) {
-                most(R.a[0], *(const float4*)(dm + GQ_KS * s + kq), mxm);
-                most(R.a[1], *(const float4*)(dm + GQ_KS * s + 32 + kq), mxm);
-            }
-        }
-        auto exponent = [&](float v) {  // S with |x|·2^S < 2^30
-            v = fmaxf(v, aeth_dpp_xor1f(v));
-            v = fmaxf(v, aeth_dpp_xor2f(v));
-            v = fmaxf(v, aeth_dpp_mirror8f(v));
-            int E = 0;
-            if (v > 0.0f) (void)frexpf(v, &E);
-            return 30 - E;
-        };
-        int any = bad ? 1 : 0;
-        any |= aeth_dpp_xor1(any);
-        any |= aeth_dpp_xor2(any);
-        any |= __builtin_amdgcn_mov_dpp(any, 0x141, 0xF, 0xF, false);
-        Srow = exponent(mx);
-        if (MIN) Srowm = exponent(mxm);
-        if ((tid & 7) == 0) {
-            Sx[0][rr] = any ? GQ_BAD : Srow;
-            if (MIN) Sx[MIN ? 1 : 0][rr] = Srowm;
-        }
-    }
-
     const int mt = wave & 1, cp = wave >> 1;  // this wave's 32 rows, and column tiles 2cp, 2cp + 1
     i32x16 acc[2][4];
 #pragma unroll
@@ -280,7 +253,7 @@ __global__ void __launch_bounds__(512) k_gq_gemm(GqArgs G) {
         for (int q = 0; q < 4; q++) acc[c][q] = (i32x16){};
     {
         const i32x4* vb = (const i32x4*)(G.v + (int64_t)B * G.kp * 256) + 2 * cp * 64 + lane;  // + (2s + j)·512 + 64·c
-        Raw P, Q;
+        GqRaw P, Q;
         i32x4 b0[2][2], b1[2][2];
         const int last = s1 - 1;
         auto loadB = [&](int s, i32x4 (&o)[2][2]) {
@@ -304,7 +277,7 @@ __global__ void __launch_bounds__(512) k_gq_gemm(GqArgs G) {
         };
         // step s: its digits are in `cur`; of a SIMD's waves w and w + 4 one multiplies while the other converts step
         // s + 1 (past the last one into a buffer nobody reads). The loads run two steps ahead.
-        auto step = [&](int s, const uint8_t* cur, uint8_t* nxt, i32x4 (&b)[2][2], Raw& R) {
+        auto step = [&](int s, const uint8_t* cur, uint8_t* nxt, i32x4 (&b)[2][2], GqRaw& R) {
             __syncthreads();  // cur is written, and nxt read by every wave
             if (wave < 4) product(cur, b);
             __builtin_amdgcn_sched_barrier(0);
@@ -332,7 +305,7 @@ __global__ void __launch_bounds__(512) k_gq_gemm(GqArgs G) {
         const i32x4* vb = (const i32x4*)(G.mins + (int64_t)B * G.kp * 32) + lane;
         const int q = wave >> 1;
         i32x16 am = (i32x16){};
-        Raw R;
+        GqRaw R;
         loadA(s0, dm, R);
         __syncthreads();  // the main loop's operands are read
         convert(R, Srowm, dig[0]);
@@ -353,6 +326,7 @@ __global__ void __launch_bounds__(512) k_gq_gemm(GqArgs G) {
         __syncthreads();
     }
     const int64_t mn = (int64_t)G.m * G.n;
+    constexpr int LB = LOW ? GQ_LOW : 0;
 #pragma unroll
     for (int c = 0; c < 2; c++)
 #pragma unroll
@@ -360,19 +334,22 @@ __global__ void __launch_bounds__(512) k_gq_gemm(GqArgs G) {
             const int lr = 32 * mt + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), cr = m0 + lr;
             const int ce = 32 * (2 * cp + c) + (lane & 31);  // output within the block
             if (cr >= G.m) continue;
-            const int S = Sx[0][lr];
+            const int S = sh.Sx[0][lr];
             double v = fma((double)acc[c][3][r], 16777216.0,
                            fma((double)acc[c][2][r], 65536.0, fma((double)acc[c][1][r], 256.0, (double)acc[c][0][r])));
-            v = ldexp(F == AETH_DTYPE_Q3_K ? -v : v, -S);
+            v = ldexp(F == AETH_DTYPE_Q3_K ? 0.0 - v : v, -S - LB);
             if constexpr (MIN) {
                 const int* p = msum + lr * 16 + (ce >> 4);
                 v -= ldexp(fma((double)p[3072], 16777216.0, fma((double)p[2048], 65536.0, fma((double)p[1024], 256.0, (double)p[0]))),
-                           -Sx[MIN ? 1 : 0][lr]);
+                           -sh.Sx[1][lr] - LB);
             }
-            if (S == GQ_BAD) {  // rare: element by element in f64
-                v = 0.0;
-                const int i1 = min(GQ_KS * s1, G.k);
-                for (int i = GQ_KS * s0; i < i1; i++) {
+            const int64_t col = 256LL * B + ce;
+            double* part = G.part + ks * mn + (int64_t)cr * G.n + col;
+            if (LOW) v += *part;
+            if (S >= GQ_NAN && !more) {  // rare: element by element in f64
+                v = S == GQ_NAN ? __builtin_nan("") : 0.0;
+                const int i1 = S == GQ_NAN ? 0 : min(GQ_KS * s1, G.k);
+                for (int i = GQ_KS * s0; i < i1 && v == v; i++) {
                     const int8_t q = G.v[((int64_t)B * G.kp + (i & ~31)) * 256 + ((ce >> 5) * 64 + (ce & 31) + 32 * ((i >> 4) & 1)) * 16 + (i & 15)];
                     double w = (double)ds[i] * (double)(F == AETH_DTYPE_Q3_K ? -(int)q : (int)q);
                     if constexpr (MIN)
@@ -381,14 +358,103 @@ __global__ void __launch_bounds__(512) k_gq_gemm(GqArgs G) {
                     v += (double)G.A[(int64_t)cr * G.k + i] * w;
                 }
             }
-            const int64_t col = 256LL * B + ce;
-            if (G.ksplit > 1) {
-                G.part[ks * mn + (int64_t)cr * G.n + col] = v;
+            if (G.ksplit > 1 || more) {
+                *part = v;
             } else {
                 float* dst = G.C + (int64_t)cr * G.ldc + col;
                 *dst = G.accumulate ? *dst + (float)v : (float)v;
             }
         }
+}
+
+template <int F, bool AL16>
+__global__ void __launch_bounds__(512) k_gq_gemm(GqArgs G) {
+    constexpr bool MIN = Gq<F>::MIN;
+    __shared__ __attribute__((aligned(16))) GqShared sh;
+    __shared__ int msum[MIN ? 4 * 64 * 16 : 1];
+    const int tid = threadIdx.x;
+    // the XCDs take workgroup ids round robin: each gets a contiguous run of tiles, the row tiles of a block column
+    // next to each other, so that an XCD reads its part of v once
+    const int T = G.gm * G.nB, ks = blockIdx.x / T, id = blockIdx.x - ks * T;
+    const int tile = (T & 7) == 0 ? (id & 7) * (T >> 3) + (id >> 3) : id;
+    const int tm = tile % G.gm, B = tile / G.gm, m0 = 64 * tm;
+    const int nst = G.kp / GQ_KS, s0 = nst * ks / G.ksplit, s1 = nst * (ks + 1) / G.ksplit;
+
+    int Srow, Srowm = 0;
+    bool wide = false;
+    {  // max |A·d| of the row over this workgroup's inputs: the row's eight threads are neighbouring lanes
+        const int rr = tid >> 3, row = min(m0 + rr, G.m - 1), kq = 4 * (tid & 7);
+        const float* a_src = G.A + (int64_t)row * G.k;
+        const float* ds = G.d + (int64_t)B * G.kp;
+        const float* dm = G.dmin + (int64_t)B * G.kp;
+        float mx = 0.0f, mxm = 0.0f;
+        // sums of four: the upper halves of their bits (2^7·(log2 + 127), about) summed, and how many are not zero
+        uint32_t lg = 0, lgm = 0;
+        int nz = 0, nzm = 0;
+        bool bad = false;
+        auto most = [&](const float4& a, const float4& d, float& m, uint32_t& lg, int& nz) {
+            const float x = fmaxf(fmaxf(fabsf(a.x * d.x), fabsf(a.y * d.y)), fmaxf(fabsf(a.z * d.z), fabsf(a.w * d.w)));
+            const float t = fabsf(a.x * d.x) + fabsf(a.y * d.y) + fabsf(a.z * d.z) + fabsf(a.w * d.w);
+            bad |= !(t < INFINITY);  // a NaN or an infinity among them (or four products near overflow)
+            lg = __builtin_amdgcn_udot2(__builtin_bit_cast(u16x2, t), (u16x2){0, 1}, lg, false);
+            nz += t > 0.0f ? 1 : 0;
+            m = fmaxf(m, x);
+        };
+#pragma unroll 4
+        for (int s = s0; s < s1; s++) {
+            GqRaw R;
+            gq_load<AL16>(G, a_src, ds, s, kq, R);
+            most(R.a[0], R.d[0], mx, lg, nz);
+            most(R.a[1], R.d[1], mx, lg, nz);
+            if constexpr (MIN) {
+                most(R.a[0], *(const float4*)(dm + GQ_KS * s + kq), mxm, lgm, nzm);
+                most(R.a[1], *(const float4*)(dm + GQ_KS * s + 32 + kq), mxm, lgm, nzm);
+            }
+        }
+        auto sum8 = [](int v) {
+            v += aeth_dpp_xor1(v);
+            v += aeth_dpp_xor2(v);
+            return v + __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, false);
+        };
+        bool far = false;  // past what the second product holds too
+        auto exponent = [&](float v, uint32_t lg, int nz) {  // S with |x|·2^S < 2^30
+            v = fmaxf(v, aeth_dpp_xor1f(v));
+            v = fmaxf(v, aeth_dpp_xor2f(v));
+            v = fmaxf(v, aeth_dpp_mirror8f(v));
+            const int over = (int)(__float_as_uint(v) >> 16), sum = sum8((int)lg), n = sum8(nz);
+            wide |= (over - 5 * 128) * n > sum;
+            far |= (over - (5 + GQ_LOW) * 128) * n > sum;
+            int E = 0;
+            if (v > 0.0f) (void)frexpf(v, &E);
+            return 30 - E;
+        };
+        Srow = exponent(mx, lg, nz);
+        if (MIN) Srowm = exponent(mxm, lgm, nzm);
+        bad = sum8(bad ? 1 : 0) != 0;
+        bool nan = false;
+        if (bad) {
+            wide = false;
+            for (int s = s0; s < s1; s++) {
+                GqRaw R;
+                gq_load<AL16>(G, a_src, ds, s, kq, R);
+#pragma unroll
+                for (int j = 0; j < 2; j++) nan |= R.a[j].x != R.a[j].x || R.a[j].y != R.a[j].y || R.a[j].z != R.a[j].z || R.a[j].w != R.a[j].w;
+            }
+            nan = sum8(nan ? 1 : 0) != 0;
+        }
+        if ((tid & 7) == 0) {
+            sh.Sx[0][rr] = nan ? GQ_NAN : bad || far ? GQ_BAD : Srow;
+            if (MIN) sh.Sx[1][rr] = Srowm;
+        }
+    }
+    wide = __builtin_amdgcn_readfirstlane(__syncthreads_or(wide));
+    gq_product<F, AL16, false>(G, tid, m0, B, ks, s0, s1, Srow, Srowm, wide, sh, msum);
+    if (wide) {
+        int t = tid;  // the second product's addresses are formed anew: nothing of it stays in registers through the first
+        asm volatile("" : "+v"(t));
+        __syncthreads();
+        gq_product<F, AL16, true>(G, t, m0, B, ks, s0, s1, Srow, Srowm, false, sh, msum);
+    }
 }
 
 bool aeth_gq_gemm_rows(const aeth_weight* w, int64_t m) {
@@ -417,7 +483,7 @@ int aeth_gemm_gq_launch(const aeth_weight* w, const float* d_a, int64_t m, float
     if (T * ksplit > (1LL << 22) || uw > (1LL << 23))
         return aeth_set_error(AETH_EINVAL, "gemm q2_k/q3_k: shape too large");
     const int64_t vb = gq_up(nB * kp * 256), db = gq_up(nB * kp * 4), mb = gq_up(nB * kp * 32);
-    const int64_t pb = ksplit > 1 ? ksplit * m * w->n * 8 : 0;
+    const int64_t pb = ksplit * m * w->n * 8;  // (with K whole, for a first of two products)
     void* ws = nullptr;
     int rc = aeth_stream_scratch(s, AETH_SCRATCH_DEQ, (size_t)(vb + db + (q2 ? mb + db : 0) + pb), &ws);
     if (rc) return rc;

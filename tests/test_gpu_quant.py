@@ -941,6 +941,67 @@ def test_gguf_int8_gemm_edges(gpu, dtype, m, n, k):
     assert np.isnan(bad[m - 1]).all() and np.array_equal(bad[1:m - 1], got[1:m - 1])
 
 
+# inputs of a row far above the others, by what factor: in the activations (row i takes the i-th set), or in the block
+# scales of one input (None)
+FAR = [{5: 1e3}, {17: 1e4}, {300: 1e5}, {511: 1e6}, {0: 1e8}, {64: 1e30}, {3: -1e5, 4: 1e5, 400: 1e4, 401: 300.0},
+       {i: 1e6 for i in range(20, 30)}, {7 * i: 1000.0 ** (i + 1) for i in range(11)}, {i: 3e5 for i in range(0, 500, 50)}]
+
+
+@pytest.mark.parametrize("dtype", [Q2_K, Q3_K])
+@pytest.mark.parametrize("m,n,k,scales", [(33, 512, 1100, False), (70, 256, 4096, False), (40, 768, 640, True),
+                                            (40, 768, 320, False)])
+def test_gguf_int8_gemm_far_values(gpu, dtype, m, n, k, scales):
+    """One activation or block scale 10^3 .. 10^33 times the others of its row, whose integer weights are 0 in every other
+    block: the outputs there keep the precision of the rest of the row. A product is off by at most 1.5 units, and a unit is at
+    most 2^-24 of the geometric mean of the sums of four products of its row, block and K part, so at most 2^-22 of their
+    mean (twice that for the mean of a part against the whole row's): 3·2^-22·mean|A·d|·Σ|v|, without the far values,
+    beside the rounding of the result (and, Q2_K, of the reference's weights). Plain and accumulate, K split and whole."""
+    torch = gpu
+    be, bb = GEOM[dtype]
+    raw = synth_blocks(dtype, n * k // be, m + n + k).reshape(k, n // 256, bb)
+    sc, ats = (slice(4, 20), (0, 2)) if dtype == Q2_K else (slice(96, 108), (108,))
+    zero = 0 if dtype == Q2_K else np.array([0] * 8 + [0xAA] * 4, np.uint8)  # Q2_K: sc = m = 0; Q3_K: sc − 32 = 0
+    x = np.random.default_rng(m * n).standard_normal((m, k)).astype(np.float32)
+    x[:, ::9] = 0.0
+    x[m - 1, 64:] = 0.0  # a sparse row
+    far = np.zeros((m, k), bool)
+    if scales:
+        for i in (1, 200, 639):
+            raw[i, ::2, ats[0]:ats[0] + 2] = np.array([30000.0], np.float16).view(np.uint8)
+            raw[i, ::2, sc] = zero
+            far[:, i] = True
+    else:
+        for r in range(m - 1):
+            for i, f in FAR[r % len(FAR)].items():
+                if i >= k:
+                    continue
+                x[r, i] = np.float32(f)
+                raw[i, ::2, sc] = zero
+                far[r, i] = True
+    raw = raw.reshape(-1)
+    w = make_weight(torch, dtype, n, k, raw)
+    got = gemv(torch, w, x, n, m).astype(np.float64)
+    acc = gemv(torch, w, x, n, m, A.MM_ACCUMULATE, np.random.default_rng(k).standard_normal(m * n)).astype(np.float64)
+    A.lib().aeth_weight_free(w)
+    x64, w64 = x.astype(np.float64), O.dequant(dtype, raw, n * k).astype(np.float64).reshape(k, n)
+    ref = x64 @ w64
+    bound = 2.0 ** -24 * np.abs(ref) + (2.0 ** -24 * (np.abs(x64) @ np.abs(w64)) if dtype == Q2_K else 0.0)
+    blocks = raw.reshape(k, n // 256, bb)
+    for at in ats:
+        d = blocks[:, :, at:at + 2].copy().view(np.float16)[:, :, 0].astype(np.float64)  # [k][n / 256]
+        for b in range(n // 256):
+            p = np.abs(x64 * d[:, b]) * ~far
+            mean = p.sum(1) / np.maximum(1, (p > 0).sum(1))
+            vmax = 45 if dtype == Q2_K and at == 0 else 15 if dtype == Q2_K else 128
+            # Σ|v| over the nonzero products, from the weights: |v| <= vmax, and for Q3_K |w| / d exactly
+            cols = slice(256 * b, 256 * b + 256)
+            v = np.abs(w64[:, cols]) / np.where(d > 0, d, 1.0)[:, b:b + 1] if dtype == Q3_K else np.full((k, 256), float(vmax))
+            bound[:, cols] += 3 * 2.0 ** -22 * mean[:, None] * ((p > 0).astype(np.float64) @ v)
+    assert (np.abs(got - ref) <= bound).all()
+    y0 = np.random.default_rng(k).standard_normal(m * n).astype(np.float32).reshape(m, n)
+    assert (np.abs(acc - (ref + y0)) <= bound + 2.0 ** -24 * np.abs(ref + y0)).all()
+
+
 @pytest.mark.parametrize("m,n,k", [(32, 4, 32), (33, 132, 96), (65, 300, 544), (64, 128, 4096), (130, 1028, 1056),
                                    (300, 5124, 64)])
 def test_gemm_f16_tiles_scales_infinities(gpu, m, n, k):
