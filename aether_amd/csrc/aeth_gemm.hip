@@ -821,11 +821,16 @@ int aeth_gemm_f16_launch(const aeth_weight* w, const float* d_a, int64_t m, floa
     const int64_t mp = aeth_cdiv(m, G2_BM) * G2_BM, gm = mp / G2_BM, gn = aeth_cdiv(w->n, G2_BN);
     _Float16 *frag, *Sh;
     float* esc;
+    void* ws = nullptr;
+    SplitPlan P;  // each wave keeps at least 16 slices, the 256 elements of a K-quant super-block
+    if (!aeth_stream_scratch_try(s, AETH_SCRATCH_GEMM, (size_t)aeth_gemm_ws_bytes(m, k), &ws)) return AETH_NO_SCRATCH;
+    if (split_plan(s, gm, gn, k / 2048, false, P)) {
+        (void)hipGetLastError();
+        return AETH_NO_SCRATCH;
+    }
     // the dot-product mode does not exist for F16: its flag is ignored
     int rc = gemm_prep(d_a, m, k, flags & ~AETH_MM_Q8_ACTIVATIONS, nullptr, s, nullptr, 0, frag, Sh, esc, true);
     if (rc) return rc;
-    SplitPlan P;  // each wave keeps at least 16 slices, the 256 elements of a K-quant super-block
-    if ((rc = split_plan(s, gm, gn, k / 2048, false, P))) return rc;
     const int c16 = ((uintptr_t)d_c & 15) == 0 && (ldc & 3) == 0;
     F16Args Q{(const uint8_t*)frag, esc, w->p0, (int)m, (int)w->n, k, (int)mp, (int)gm, (int)gn, (int)(mp * k * 4),
               (int)w->bytes, d_c, ldc, (flags & AETH_MM_ACCUMULATE) ? 1 : 0, 0, c16, P.ksplit, P.part,

@@ -461,6 +461,8 @@ bool aeth_gq_gemm_rows(const aeth_weight* w, int64_t m) {
     if (!w || (w->dtype != AETH_DTYPE_Q2_K && w->dtype != AETH_DTYPE_Q3_K) || w->order != AETH_ORDER_GGUF) return false;
     // whole blocks per input; i32 sums of 2^14 a product; one row's offsets in an int
     if (w->n % 256 != 0 || w->k < 4 || w->k > 65536 || w->n > (1LL << 28) || m > (1LL << 20)) return false;
+    // grids below 2^32 threads (a larger product goes on as blocks that straddle inputs do)
+    if (aeth_cdiv(m, 64) * (w->n / 256) > (1LL << 22) || w->n / 256 * aeth_cdiv(w->k, GQ_KS) > (1LL << 23)) return false;
     // k_colk reads the weight once per 8 rows; this product costs about the same up to 64. At 8 / 16 / 24 rows, here
     // against there: Q3_K 4096 × 4096 35 / 37 / 36 µs and 21 / 28 / 36, 14336 × 4096 (from 40 million weights on)
     // 55 / 57 / 59 and 39 / 64 / 85; Q2_K 4096 × 4096 - / 42 / 40 and - / 29 / 38, 14336 × 4096 at 16 rows 74 and 68.
@@ -480,13 +482,10 @@ int aeth_gemm_gq_launch(const aeth_weight* w, const float* d_a, int64_t m, float
     // K split over workgroups while they all fit the chip at once, at least 4 steps each
     const int64_t ksplit = std::max<int64_t>(1, std::min<int64_t>(aeth_num_cus() / T, kp / (4 * GQ_KS)));
     const int64_t uw = nB * (kp / GQ_KS);
-    if (T * ksplit > (1LL << 22) || uw > (1LL << 23))
-        return aeth_set_error(AETH_EINVAL, "gemm q2_k/q3_k: shape too large");
     const int64_t vb = gq_up(nB * kp * 256), db = gq_up(nB * kp * 4), mb = gq_up(nB * kp * 32);
     const int64_t pb = ksplit * m * w->n * 8;  // (with K whole, for a first of two products)
     void* ws = nullptr;
-    int rc = aeth_stream_scratch(s, AETH_SCRATCH_DEQ, (size_t)(vb + db + (q2 ? mb + db : 0) + pb), &ws);
-    if (rc) return rc;
+    if (!aeth_stream_scratch_try(s, AETH_SCRATCH_DEQ, (size_t)(vb + db + (q2 ? mb + db : 0) + pb), &ws)) return AETH_NO_SCRATCH;
     uint8_t* p = (uint8_t*)ws;
     GqArgs G{};
     G.raw = w->p0; G.A = d_a; G.m = (int)m; G.n = (int)w->n; G.k = (int)w->k; G.kp = (int)kp; G.nB = (int)nB;

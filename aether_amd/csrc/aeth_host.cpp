@@ -59,6 +59,12 @@ int aeth_stream_scratch(hipStream_t s, int use, size_t bytes, void** out) {
     return AETH_OK;
 }
 
+bool aeth_stream_scratch_try(hipStream_t s, int use, size_t bytes, void** out) {
+    if (aeth_stream_scratch(s, use, bytes, out) == AETH_OK) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 void aeth_stream_scratch_release(hipStream_t s) {
     aeth_blas_release_stream(s);
     std::lock_guard<std::mutex> lk(g_scratch_mu);
@@ -104,8 +110,15 @@ int aeth_qmatmul_ld(const aeth_weight* w, const float* d_a, int64_t m, float* d_
     if (m > 1 && aeth_q5k_gemm_rows(w, m)) return aeth_gemm_q4k_launch(w, d_a, m, d_c, flags, s, ldc);  // Q5_K
     if (m > 1 && aeth_q6k_gemm_rows(w, m)) return aeth_gemm_q6k_launch(w, d_a, m, d_c, flags, s, ldc);  // Q6_K
     if (m > 1 && aeth_q80_gemm_rows(w, m)) return aeth_gemm_q80_launch(w, d_a, m, d_c, flags, s, ldc);  // Q8_0
-    if (m > 1 && aeth_gq_gemm_rows(w, m)) return aeth_gemm_gq_launch(w, d_a, m, d_c, flags, s, ldc);
-    if (m > 1 && aeth_f16_gemm_rows(w, m)) return aeth_gemm_f16_launch(w, d_a, m, d_c, flags, s, ldc);
+    // (these two leave a call to what follows where their scratch cannot be had: under graph capture, or out of memory)
+    if (m > 1 && aeth_gq_gemm_rows(w, m)) {
+        const int rc = aeth_gemm_gq_launch(w, d_a, m, d_c, flags, s, ldc);
+        if (rc != AETH_NO_SCRATCH) return rc;
+    }
+    if (m > 1 && aeth_f16_gemm_rows(w, m)) {
+        const int rc = aeth_gemm_f16_launch(w, d_a, m, d_c, flags, s, ldc);
+        if (rc != AETH_NO_SCRATCH) return rc;
+    }
     // the other block formats from a few hundred rows on: dequantized once, one DGEMM (instead
     // of the weight streamed once per row by the batched GEMV). Their dequantized
     // weights are finite (K-quant scales go through decode_d), so the SGEMM's

@@ -214,6 +214,10 @@ enum {
     AETH_SCRATCH_SPLIT = 6, // partial output tiles of a GEMM split over K across workgroups (aeth_gemm.hip)
 };
 int aeth_stream_scratch(hipStream_t s, int use, size_t bytes, void** out);
+// The same for a caller that has another way: false, and HIP's error cleared, where it cannot be had. A launch that
+// leaves its call to that other way returns AETH_NO_SCRATCH, having enqueued nothing.
+bool aeth_stream_scratch_try(hipStream_t s, int use, size_t bytes, void** out);
+constexpr int AETH_NO_SCRATCH = 1;
 // Frees every scratch buffer of stream s (before the stream is destroyed).
 void aeth_stream_scratch_release(hipStream_t s);
 // Resolves the device address of the no-allocation entry point's static

@@ -147,8 +147,10 @@ AETH_API int aeth_load_quant(int dtype, const void* d_src, int64_t k, int64_t n,
  * stream), as do the rocBLAS handles: calls on different streams never share
  * them, calls on one stream run in order. A buffer grows on first use of a
  * larger shape (a grow waits for the stream and fails with AETH_ESTATE during
- * graph capture: run every shape once before capturing). Several host
- * threads enqueueing on the same stream at once must serialise their calls. */
+ * graph capture: run every shape once before capturing; a GGUF-order Q2_K,
+ * Q3_K or F16 batch whose GEMM's buffers cannot be had takes the row-batched
+ * kernel or the DGEMM where theirs can). Several host threads enqueueing on
+ * the same stream at once must serialise their calls. */
 AETH_API int aeth_qmatmul(const aeth_weight* w, const float* d_a, int64_t m, float* d_c, unsigned flags,
                           void* stream);
 

@@ -1049,6 +1049,51 @@ def test_gemm_f16_tiles_scales_infinities(gpu, m, n, k):
     L.aeth_weight_free(w)
 
 
+# a smaller batch of a larger weight leaves the row-batched kernel enough scratch, the GEMMs' own was never allocated
+@pytest.mark.parametrize("dtype,warm,m,n,k", [(Q3_K, (24, 8192), 25, 4096, 1024), (Q2_K, (24, 8192), 28, 4096, 1024),
+                                              (F16, (8, 12288), 32, 4096, 1024)])
+def test_batch_under_capture_without_gemm_scratch(gpu, dtype, warm, m, n, k):
+    """Under graph capture no scratch can grow: a batch whose GEMM would need one takes the row-batched kernel when
+    that has all it needs. Replayed with other work between, each replay gives the product of the present inputs."""
+    torch = gpu
+    L = A.lib()
+    rng = np.random.default_rng(dtype + m)
+    s = torch.cuda.Stream()
+    st = ctypes.c_void_p(s.cuda_stream)
+    ws = []
+    for nn in (warm[1], n):
+        ws.append((nn, weight_gguf(dtype, nn, k, dtype + nn)))
+    hs = [make_weight(torch, dtype, nn, k, raw) for nn, raw in ws]
+    x, y = torch.zeros(m, k, device="cuda"), torch.zeros(m, n, device="cuda")
+    big = torch.zeros(warm[0], warm[1], device="cuda")
+    torch.cuda.synchronize()
+    A.check(L.aeth_qmatmul(hs[0], x.data_ptr(), warm[0], big.data_ptr(), 0, st), "warm")
+    s.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        A.check(L.aeth_qmatmul(hs[1], x.data_ptr(), m, y.data_ptr(), 0, st), "captured")
+    w64 = O.dequant(dtype, ws[1][1], n * k).astype(np.float64).reshape(k, n)
+    for i in range(3):
+        xh = rng.standard_normal((m, k)).astype(np.float32)
+        x.copy_(torch.from_numpy(xh))
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        # chains of at most k/8 + 1 fused multiply-adds a wave, a tree and an f64 sum; Q2_K's weights rounded once more
+        bound = (k / 8 + 8) * 2.0 ** -24 * (np.abs(xh).astype(np.float64) @ np.abs(w64))
+        assert (np.abs(y.cpu().numpy() - xh.astype(np.float64) @ w64) <= bound).all(), i
+        A.check(L.aeth_qmatmul(hs[0], x.data_ptr(), warm[0], big.data_ptr(), 0, st), "between")
+        torch.cuda.synchronize()
+    for h in hs:
+        L.aeth_weight_free(h)
+
+
+def weight_gguf(dtype, n, k, seed):
+    """A weight in the file's [k][n] order."""
+    return synth_blocks(dtype, n * k // GEOM[dtype][0], seed)
+
+
 def test_gguf_order_zero_activation_skips_infinite_weights(gpu):
     """A zero activation skips its weight row even when that row holds an
     infinity (0·inf would be NaN): matmul_f32_gguf's `if scale != 0.0`."""
