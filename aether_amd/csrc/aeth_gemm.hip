@@ -61,9 +61,11 @@
 
 // ── activation prep (f32 A [m][k]; rows m..mp-1 read as zero). Writes
 //  * escale[r] = 2^e, e = 0 if 2^-3 <= max |A[r]| < 2^14, else the least (from −100 on)
-//    with |A[r]·2^-e| < 2^14 (INF, the F16 product's: always that, as its weights are no
-//    integers, and an infinite element gives hi = ±Inf, lo = 0 and is left out of the maximum;
-//    as a test of every element at run time that cost the other GEMMs 1.5 % of their time);
+//    with |A[r]·2^-e| < 2^14. F16W, the F16 product's (a template argument: a test at run time of
+//    every element cost the other GEMMs 1.5 % of their time): always that, and −1 with zero
+//    fragments for a row that the kernel sums in f64 instead: one with an infinity, or whose largest
+//    value is 2^13 above the geometric mean of the sums of eight, so that most values lie below
+//    2^-16 of it, where the parts leave less than 22 bits;
 //  * fragment (mt, ks, part) = 1 KiB at ((mt·nks + ks)·2 + part)·1024 bytes
 //    (nks = k/16): lane l holds row 32·mt + l%32 at k-positions
 //    16·ks + 8·(l/32) + perm4(i), i < 8, of A·2^-e, part 0 = hi, 1 = lo;
@@ -123,12 +125,12 @@ __device__ __forceinline__ void prep_ld8(const float* __restrict__ p, float* v) 
 // SPW: steps a wave holds in registers, at least its share ⌈S/4⌉ (1, 2, 4 or 8: k ≤ 16384 in one chunk).
 // PREP_ROWS: rows per workgroup, 4 (2 where the producer's 8 steps of inputs need more than the
 // 128 registers of a 16-wave workgroup; 1 for at most 128 rows, which then take more CUs).
-template <bool AL16, bool Q8, int MODE, int SPW, int PREP_ROWS, bool INF>
+template <bool AL16, bool Q8, int MODE, int SPW, int PREP_ROWS, bool F16W>
 __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs P) {
     static_assert(!Q8 || MODE == PREP_PLAIN, "the producers feed the exact mode");
     constexpr int WK = PREP_WK;
     __shared__ __attribute__((aligned(16))) uint4 stage[WK][2][64][PREP_LD];  // [part j][hi/lo][group][row]
-    __shared__ float red[2][PREP_ROWS * WK];
+    __shared__ float red[F16W ? 4 : 2][PREP_ROWS * WK];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, ri = wv % PREP_ROWS, j = wv / PREP_ROWS;
     const int r0 = blockIdx.x * PREP_ROWS, r = r0 + ri;
     const bool live = r < P.m;
@@ -178,6 +180,7 @@ __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs
     };
     const int nck = (nsmax + SPW - 1) / SPW;  // chunks (1 unless a plain row is longer than 16384)
     float mx = 0.0f;
+    int lg = 0, nz = 0;  // F16W: sums of eight, the upper halves of their bits (2^7·(log2 + 127), about) and how many are not 0
     for (int c = 0; c < nck; c++) {
         load(c * SPW);
         if (MODE == PREP_RMSNORM) {  // rms = sqrt(Σx²/k + eps); x ← (x / rms)·w (one chunk: k ≤ 16384)
@@ -205,20 +208,46 @@ __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs
         for (int t = 0; t < SPW; t++)
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const float av = fabsf(v[t][i]);
-                mx = fmaxf(mx, INF && av == INFINITY ? 0.0f : av);
+                mx = fmaxf(mx, fabsf(v[t][i]));
             }
+        if (F16W) {
+#pragma unroll
+            for (int t = 0; t < SPW; t++) {
+                float sum = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 8; i++) sum += fabsf(v[t][i]);
+                lg += (int)(__float_as_uint(sum) >> 16);
+                nz += __popcll(__ballot(sum > 0.0f));  // of the wave
+            }
+        }
     }
     mx = aeth_wave_max(mx);
+    float logs = 0.0f, groups = 0.0f;
+    if (F16W) {
+        logs = aeth_wave_sum((float)lg);
+        if (lane == 0) {
+            red[F16W ? 2 : 0][wv] = logs;
+            red[F16W ? 3 : 0][wv] = (float)nz;
+        }
+    }
     if (lane == 0) red[1][wv] = mx;
     __syncthreads();
     mx = 0.0f;
 #pragma unroll
     for (int q = 0; q < WK; q++) mx = fmaxf(mx, red[1][PREP_ROWS * q + ri]);
+    if (F16W) {
+        logs = groups = 0.0f;
+#pragma unroll
+        for (int q = 0; q < WK; q++) {
+            logs += red[F16W ? 2 : 0][PREP_ROWS * q + ri];
+            groups += red[F16W ? 3 : 0][PREP_ROWS * q + ri];
+        }
+    }
     int E = 14;
     if (mx > 0.0f && isfinite(mx)) (void)frexpf(mx, &E);
-    const float esc = ldexpf(1.0f, INF || E > 14 || E < -2 ? max(E - 14, -100) : 0);
-    if (j == 0 && lane == 0) P.escale[r] = esc;
+    const float esc = ldexpf(1.0f, F16W || E > 14 || E < -2 ? max(E - 14, -100) : 0);
+    const bool apart = F16W && (mx == INFINITY || ((float)(__float_as_uint(mx) >> 16) - 13 * 128.0f) * groups > logs);
+    if (j == 0 && lane == 0) P.escale[r] = apart ? -1.0f : esc;
     const float inv = 1.0f / esc;  // a power of two: the products below are exact scalings
     const int tp = tid % (64 * PREP_ROWS);  // thread of the part's PREP_ROWS waves
     for (int c = 0; c < nck; c++) {
@@ -229,6 +258,10 @@ __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs
             const int gb = 64 * (s0 + c * SPW + t), gi = gb + lane;
             const bool sl = c * SPW + t < ns;  // this part has the step (uniform per wave)
             float* x = v[t];
+            if (F16W) {
+#pragma unroll
+                for (int i = 0; i < 8; i++) x[i] = apart ? 0.0f : x[i];
+            }
             if (Q8) {  // quantize_q8_0_block (neon.rs:45-104), then the value q·f16(d)
                 int nan = 0;
                 float bm = 0.0f;
@@ -262,7 +295,7 @@ __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs
                 const float tv = x[perm4(i)] * inv;
                 const _Float16 th = (_Float16)tv;
                 hi[i] = th;
-                lo[i] = INF && fabsf(tv) == INFINITY ? (_Float16)0.0f : (_Float16)(tv - (float)th);
+                lo[i] = (_Float16)(tv - (float)th);
             }
             if (sl && gi < ng && (lane & 3) == 0) {  // gi < ng is uniform per four lanes (ng % 32 == 0)
                 const float sv = sum * inv * 0.03125f;
@@ -503,26 +536,26 @@ int64_t aeth_gemm_ws_bytes(int64_t m, int64_t k) {
     return mp * k * 2 * 2 + mp * (k / 32) * 2 * 2 + mp * 4 + 256;
 }
 
-template <bool AL16, bool Q8, int MODE, int SPW, bool INF>
+template <bool AL16, bool Q8, int MODE, int SPW, bool F16W>
 static void prep_launch_r(unsigned mp, hipStream_t s, const PrepArgs& P) {
     constexpr int R = SPW == 8 && MODE != PREP_PLAIN ? 2 : 4;
     if (mp <= 128)  // few rows: one row per workgroup, so that they spread over more CUs
-        hipLaunchKernelGGL((k_gemm_prep<AL16, Q8, MODE, SPW, 1, INF>), dim3(mp), dim3(64 * PREP_WK), 0, s, P);
+        hipLaunchKernelGGL((k_gemm_prep<AL16, Q8, MODE, SPW, 1, F16W>), dim3(mp), dim3(64 * PREP_WK), 0, s, P);
     else
-        hipLaunchKernelGGL((k_gemm_prep<AL16, Q8, MODE, SPW, R, INF>), dim3(mp / R), dim3(64 * R * PREP_WK), 0, s, P);
+        hipLaunchKernelGGL((k_gemm_prep<AL16, Q8, MODE, SPW, R, F16W>), dim3(mp / R), dim3(64 * R * PREP_WK), 0, s, P);
 }
-template <bool AL16, bool Q8, int MODE, bool INF = false>
+template <bool AL16, bool Q8, int MODE, bool F16W = false>
 static void prep_launch(int spw, unsigned mp, hipStream_t s, const PrepArgs& P) {
-    if (spw == 1) prep_launch_r<AL16, Q8, MODE, 1, INF>(mp, s, P);
-    else if (spw == 2) prep_launch_r<AL16, Q8, MODE, 2, INF>(mp, s, P);
-    else if (spw == 4) prep_launch_r<AL16, Q8, MODE, 4, INF>(mp, s, P);
-    else prep_launch_r<AL16, Q8, MODE, 8, INF>(mp, s, P);
+    if (spw == 1) prep_launch_r<AL16, Q8, MODE, 1, F16W>(mp, s, P);
+    else if (spw == 2) prep_launch_r<AL16, Q8, MODE, 2, F16W>(mp, s, P);
+    else if (spw == 4) prep_launch_r<AL16, Q8, MODE, 4, F16W>(mp, s, P);
+    else prep_launch_r<AL16, Q8, MODE, 8, F16W>(mp, s, P);
 }
 
 // The activation prep of the Q4_K and Q6_K GEMMs: A (or, with `in`, its producer's input) into
 // hi/lo fp16 MFMA fragments, sub-block sums and row scales in ws (the stream's scratch when null).
 static int gemm_prep(const float* d_a, int64_t m, int k, unsigned flags, const GemmIn* in, hipStream_t s, void* ws,
-                     size_t ws_bytes, _Float16*& frag, _Float16*& Sh, float*& esc, bool keep_inf = false) {
+                     size_t ws_bytes, _Float16*& frag, _Float16*& Sh, float*& esc, bool f16w = false) {
     const int mode = in ? in->mode : PREP_PLAIN;
     const int64_t mp = aeth_cdiv(m, G2_BM) * G2_BM;  // fragment rows: whole 64-row tiles
     if (mp > (1LL << 20) || mp * k > (1LL << 29)) return aeth_set_error(AETH_EINVAL, "gemm: m=%lld too large", (long long)m);
@@ -545,8 +578,8 @@ static int gemm_prep(const float* d_a, int64_t m, int k, unsigned flags, const G
     const int spw = share <= 1 ? 1 : share <= 2 ? 2 : share <= 4 ? 4 : 8;
     const PrepArgs P{d_a, in ? in->norm_w : nullptr, in ? in->eps : 0.0f, (int)m, k, esc, frag, Sh, Sl};
     const unsigned pg = (unsigned)mp;  // fragment rows (whole 64-row tiles)
-    if (keep_inf && al16) prep_launch<true, false, PREP_PLAIN, true>(spw, pg, s, P);
-    else if (keep_inf) prep_launch<false, false, PREP_PLAIN, true>(spw, pg, s, P);
+    if (f16w && al16) prep_launch<true, false, PREP_PLAIN, true>(spw, pg, s, P);
+    else if (f16w) prep_launch<false, false, PREP_PLAIN, true>(spw, pg, s, P);
     else if (mode == PREP_RMSNORM) prep_launch<true, false, PREP_RMSNORM>(spw, pg, s, P);
     else if (mode == PREP_SWIGLU) prep_launch<true, false, PREP_SWIGLU>(spw, pg, s, P);
     else if (al16 && q8) prep_launch<true, true, PREP_PLAIN>(spw, pg, s, P);
@@ -832,7 +865,7 @@ int aeth_gemm_f16_launch(const aeth_weight* w, const float* d_a, int64_t m, floa
     int rc = gemm_prep(d_a, m, k, flags & ~AETH_MM_Q8_ACTIVATIONS, nullptr, s, nullptr, 0, frag, Sh, esc, true);
     if (rc) return rc;
     const int c16 = ((uintptr_t)d_c & 15) == 0 && (ldc & 3) == 0;
-    F16Args Q{(const uint8_t*)frag, esc, w->p0, (int)m, (int)w->n, k, (int)mp, (int)gm, (int)gn, (int)(mp * k * 4),
+    F16Args Q{(const uint8_t*)frag, esc, w->p0, d_a, (int)m, (int)w->n, k, (int)mp, (int)gm, (int)gn, (int)(mp * k * 4),
               (int)w->bytes, d_c, ldc, (flags & AETH_MM_ACCUMULATE) ? 1 : 0, 0, c16, P.ksplit, P.part,
               (int)(gn * G2_BN), P.t_full, P.tsplit};
     return aeth_gemm_f16_kernel_launch(Q, s);

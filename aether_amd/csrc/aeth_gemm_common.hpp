@@ -303,8 +303,9 @@ int aeth_gemm_q80_kq_launch(const Q80Args& G, hipStream_t s);
 // Arguments of the F16 GEMM kernel (aeth_gemm_f16.hip): A as for KqArgs, W the [k][n] halves.
 struct F16Args {
     const uint8_t* frag;   // A·2^-e as fp16 MFMA fragments (k_gemm_prep)
-    const float* escale;   // [mp]: 2^e
+    const float* escale;   // [mp]: 2^e; −1: the row is summed in f64 from A
     const uint8_t* w;
+    const float* A;        // [m][k]
     int m, n, k, mp;
     int gm, gn;            // 64-row and 128-column tiles of C
     int a_bytes, w_bytes;  // buffer extents (each < 2^31)

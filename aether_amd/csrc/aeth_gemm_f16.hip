@@ -5,8 +5,9 @@
 // The exact mode of the Q4_K GEMM: A·2^-e split into fp16 hi/lo MFMA fragments (k_gemm_prep in
 // aeth_gemm.hip), f32 accumulation on v_mfma_f32_32x32x16_f16, two passes per product; the weights are
 // their own exact operands. The reference skips a zero activation, which matters to weights that are
-// infinite or NaN: weights holding one keep k_col (aeth_f16_gemm_rows). An infinite activation enters as
-// hi = ±Inf, lo = 0, so that its row gets the ±Inf and NaN an f32 sum gives.
+// infinite or NaN: weights holding one keep k_col (aeth_f16_gemm_rows). Rows that the two parts do not hold (an
+// infinity; a largest value far above the others) come with zero fragments and the scale −1: the epilogue puts the
+// negative of their f64 sum in place of the tile's, element by element over this workgroup's part of K.
 //
 // Work split as aeth_gemm_q80.hip: 64 × 128 workgroup tiles, 8 waves over eighths of the 16-position
 // slices (and K over several workgroups when the tiles are few). Nothing is shared between waves and
@@ -15,7 +16,7 @@
 // the eight k rows of its half (rows of 256 contiguous bytes). Operand column n of tile c is output column
 // 4n + c, so the transpose is 16 v_perm a slice and a lane ends with four neighbouring outputs.
 // What bounds it: operand bytes, 8 KiB per wave and slice (64 B per CU and clock at the full MFMA rate; the
-// L2s deliver about a third of that). m = 333, 4096 × 4096: 460 → 52 µs with the prep (43.7 µs alone);
+// L2s deliver about a third of that). m = 333, 4096 × 4096: 456 → 40.5 µs with the prep;
 // m = 512, 14336 × 4096: 1834 → 164 µs.
 #include <math.h>
 #include <stdint.h>
@@ -97,6 +98,10 @@ __global__ void __launch_bounds__(64 * F16_W) k_gemm_f16(F16Args G) {
 
     // the eight K-eighth tiles meet in LDS: wave → m-tile wave/4, result registers [4·(wave%4), +4)
     const int mt = wave >> 2, r0 = 4 * (wave & 3), lr = lane & 31, col = n0 + 4 * lr;
+    const int row0 = m0 + 32 * mt + 2 * r0 + 4 * (lane >> 5);  // row of register r0 + r: row0 + r
+    float es[4];  // in flight during the reduction
+#pragma unroll
+    for (int r = 0; r < 4; r++) es[r] = G.escale[row0 + r];
     if (wave >= 4) {
 #pragma unroll
         for (int q = 0; q < 2; q++)
@@ -118,9 +123,7 @@ __global__ void __launch_bounds__(64 * F16_W) k_gemm_f16(F16Args G) {
                 }
     }
     __syncthreads();
-    const int row0 = m0 + 32 * mt + 2 * r0 + 4 * (lane >> 5);  // row of register r0 + r: row0 + r
     float4 sum[4];
-    float es[4];
     float4 pv[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
@@ -132,6 +135,23 @@ __global__ void __launch_bounds__(64 * F16_W) k_gemm_f16(F16Args G) {
         }
         sum[r] = make_float4(v[0], v[1], v[2], v[3]);
     }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        if (es[r] < 0.0f) {  // rare (and then row0 + r < m)
+            const float* a = G.A + (int64_t)(row0 + r) * G.k;
+            const uint8_t* wc = G.w + 2 * (int64_t)min(col, G.n - 4);
+            double d[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+            for (int i = 16 * lo; i < 16 * (lo + len); i++) {
+                const uint2 h = *(const uint2*)(wc + (int64_t)i * ldw);
+                const double x = (double)a[i];
+                d[0] += x * (double)aeth_f16_to_f32(h.x & 0xFFFFu);
+                d[1] += x * (double)aeth_f16_to_f32(h.x >> 16);
+                d[2] += x * (double)aeth_f16_to_f32(h.y & 0xFFFFu);
+                d[3] += x * (double)aeth_f16_to_f32(h.y >> 16);
+            }
+            sum[r] = make_float4((float)-d[0], (float)-d[1], (float)-d[2], (float)-d[3]);
+        }
     if (nsplit > 1) {  // the split's partial tile (rows < mp, columns < pld: no bounds to check)
         int ld;
         float* P = g2_part(G.part, ks, tile, G.t_full, G.tsplit, G.gm * G.gn, G.mp, G.pld, m0, n0, ld) + 4 * lr;
@@ -141,8 +161,6 @@ __global__ void __launch_bounds__(64 * F16_W) k_gemm_f16(F16Args G) {
     }
     // n % 4 == 0: a lane's four columns are all below n or none. The loads precede the first store (it may alias).
     if (col >= G.n) return;
-#pragma unroll
-    for (int r = 0; r < 4; r++) es[r] = G.escale[row0 + r];
     if (G.accumulate) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {

@@ -1094,6 +1094,41 @@ def weight_gguf(dtype, n, k, seed):
     return synth_blocks(dtype, n * k // GEOM[dtype][0], seed)
 
 
+@pytest.mark.parametrize("m,n,k", [(33, 132, 96), (64, 4, 4096), (100, 5124, 544), (40, 256, 17408), (32, 4100, 2048)])
+def test_gemm_f16_far_values(gpu, m, n, k):
+    """Rows in which most values lie below 2^-16 of the largest (one entry 10^5 .. 10^30 times the others, and a row
+    of two such sizes), whose weights at the large entries are 0 in every third column: each output within the error of f32
+    sums of f32 products, (k/16 + 24)·2^-24·Σ|x·w|, plus 2^-22 of it for the split of the ordinary rows. No term
+    grows with the row's largest value. Through every tile remainder, K split and whole, plain, accumulate and a row with
+    an infinity among such values."""
+    torch = gpu
+    L = A.lib()
+    rng = np.random.default_rng(m + n + k)
+    wh = (rng.standard_normal((k, n)) * 0.05).astype(np.float16)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    at = rng.integers(0, k, m)
+    for r in range(m - 2):
+        x[r, at[r]] = np.float32(10.0 ** (5 + r % 26)) * (-1) ** r
+        wh[at[r], ::3] = 0
+    x[1, : k // 4] *= np.float32(1e12)
+    w = make_weight(torch, F16, n, k, wh.view(np.uint8).reshape(-1))
+    x64, w64 = x.astype(np.float64), wh.astype(np.float64)
+    ref = x64 @ w64
+    bound = (k / 16 + 24 + 4) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64))
+    bound[1] += 2.0 ** -22 * np.abs(x64[1]).max() * np.abs(w64).sum(0)
+    assert (np.abs(gemv(torch, w, x, n, m) - ref) <= bound).all()
+    y0 = rng.standard_normal((m, n)).astype(np.float32)
+    got = gemv(torch, w, x, n, m, A.MM_ACCUMULATE, y0)
+    assert (np.abs(got - (ref + y0)) <= bound + 2.0 ** -24 * np.abs(ref + y0)).all()
+    x[0, (at[0] + 1) % k] = np.inf
+    got = gemv(torch, w, x, n, m)
+    L.aeth_weight_free(w)
+    with np.errstate(invalid="ignore"):
+        inf = np.inf * w64[(at[0] + 1) % k]
+    assert np.array_equal(got[0], inf.astype(np.float32), equal_nan=True)
+    assert (np.abs(got[1:] - ref[1:]) <= bound[1:]).all()
+
+
 def test_gguf_order_zero_activation_skips_infinite_weights(gpu):
     """A zero activation skips its weight row even when that row holds an
     infinity (0·inf would be NaN): matmul_f32_gguf's `if scale != 0.0`."""
