@@ -336,6 +336,7 @@ int runner_prefill_locked(aeth_runner* r, const int32_t* tokens, int32_t n, floa
                         if ((e = aeth_rmsnorm_launch(r->p_x, attn_norm, n, d, c.rms_norm_eps, r->p_n, s))) return e;
                         normed = true;
                     }
+                    pin.prepared = false;  // this product may form its own prep in the same scratch (F16 does)
                     return aeth_qmatmul_ld(w, r->p_n, n, out, ld, 0, s);
                 }
                 pin.prepared = e == AETH_OK;

@@ -489,6 +489,24 @@ def test_runner_gguf_order_formats(gpu, mix, lm_dtype):
     assert outs[0] == outs[1]
 
 
+def test_prefill_prep_is_not_another_weights(gpu):
+    """q, k and v of three formats at 64 tokens: q's and v's GEMMs take the RMSNorm in their activation prep, formed once
+    for both, k's (F16) forms its own between them in the same scratch. The values rows do not depend on k's format."""
+    c = dict(TINY, vocab_size=64, d_model=4096, num_layers=1, num_heads=32, num_kv_heads=8, d_ff=256, max_seq_len=64)
+    L, n, v = A.lib(), 64, []
+    toks = (np.arange(n) % c["vocab_size"]).astype(np.int32)
+    for kd in (Q4_K, F16):
+        r = make_runner(build_tiny(seed=31, layer_dtype=[Q4_K, kd, Q6_K, Q4_K, Q4_K, Q4_K, Q4_K], c=c), c)
+        try:
+            A.check(L.aeth_runner_prefill(r, toks.ctypes.data, n, None, None), "prefill")
+            kv, fl = np.empty((2, c["num_kv_heads"], n, c["head_dim"]), np.float32), ctypes.c_int32()
+            A.check(L.aeth_runner_kv_to_host(r, kv.ctypes.data, ctypes.byref(fl)), "kv_to_host")
+        finally:
+            L.aeth_runner_free(r)
+        v.append(kv[1])
+    assert np.isfinite(v[0]).all() and np.array_equal(v[0], v[1])
+
+
 # The step's results reach pageable memory through the runner's pinned buffer and pinned memory directly;
 # either output may be NULL. The same prompt and step give the same bytes each way.
 @pytest.mark.parametrize("vocab", [3, 512, 1283])
