@@ -18,6 +18,8 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <mutex>
+
 #include "aeth_common.hpp"
 #include "aeth_gemm_common.hpp"
 #include "aeth_internal.hpp"
@@ -835,6 +837,9 @@ __global__ void __launch_bounds__(512, 2) k_attn_prefill_sp(const float* __restr
 // 48.0 / 59.6, 768 54 / 69.6, 1000 66 / 109, 2000 126 / 330, 4000 466 / 1318; 16 / 8 heads, n = 1000 (64) 62 / 57.
 // It needs a scratch of 32 KiB per KV head and 32 keys, the stream's own; under graph capture, where that could not grow
 // and a recorded address would not outlive a later growth, and where there is no memory for it, the f32 kernel runs.
+// Two host threads may call on one stream: from the fetch of the scratch to the launch that reads it a call holds a
+// lock, or another's fragments (or a growth that frees the buffer) could come between its two kernels.
+static std::mutex g_split_mu;
 template <int G>
 static bool attn_split_launch(const float* qkv, int64_t stride, const float* layer_kv, int64_t n, int64_t nh, int64_t nkv,
                               int64_t max_seq, int win, float* out, hipStream_t s, int* rc) {
@@ -842,13 +847,15 @@ static bool attn_split_launch(const float* qkv, int64_t stride, const float* lay
     const int64_t nqb = aeth_cdiv(n, 128 / G), wgs = nkv * aeth_cdiv(nqb, 2), nt = aeth_cdiv(n, 32);
     if (wgs < 80) return false;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return false;
-    const int64_t fb = nkv * nt * SP_TILE;
-    void* ws = nullptr;
-    if (aeth_stream_scratch(s, AETH_SCRATCH_PATTN, (size_t)(fb + nkv * nt * sizeof(int2)), &ws) != AETH_OK) {
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
+    if (cs != hipStreamCaptureStatusNone) return false;
+    const int64_t fb = nkv * nt * SP_TILE;
+    void* ws = nullptr;
+    std::lock_guard<std::mutex> lk(g_split_mu);
+    if (!aeth_stream_scratch_try(s, AETH_SCRATCH_PATTN, (size_t)(fb + nkv * nt * sizeof(int2)), &ws)) return false;
     int2* ex = (int2*)((uint8_t*)ws + fb);
     hipLaunchKernelGGL(k_attn_split, dim3((unsigned)(nkv * nt)), dim3(256), 0, s, layer_kv, (int)n, (int)nkv, max_seq, (int)nt,
                        (uint8_t*)ws, ex);

@@ -248,7 +248,13 @@ AETH_API int aeth_attn_decode_noalloc(const float* d_q, const float* d_layer_kv,
 /* Causal GQA attention of a prompt batch (attention_batch, runner.rs:1809-1883):
  * query i (row i of d_q, [n][q_stride] with head h at column h*head_dim, RoPE
  * already applied) attends to cache slots 0..i of the layer slice d_layer_kv
- * ([2][kv_heads][max_seq][head_dim]); d_out is [n][n_heads*head_dim]. */
+ * ([2][kv_heads][max_seq][head_dim]); d_out is [n][n_heads*head_dim].
+ * Long prompts (from 640 tokens on at 32 / 8 heads) lay K and V out in a buffer
+ * the library keeps per (device, stream), 32 KiB per KV head and 32 keys, which
+ * grows on first use of a longer prompt (a grow waits for the stream). Under
+ * graph capture, and where there is no memory for it, the same attention runs
+ * in f32 without it: within the error of either, not the same bits. Several
+ * host threads may call on one stream. */
 AETH_API int aeth_attn_prefill(const float* d_q, int64_t q_stride, const float* d_layer_kv, int64_t n,
                                int64_t n_heads, int64_t kv_heads, int64_t head_dim, int64_t max_seq, float* d_out,
                                void* stream);

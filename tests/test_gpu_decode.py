@@ -2,6 +2,7 @@
 the CPU oracle's restatement of runner.rs (rmsnorm, RoPE, attention, SiLU,
 argmax, one full decode step)."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -280,6 +281,48 @@ def test_attn_prefill_split_matches_f64(gpu, n, nh, nkv, max_seq):
     assert below.all()
     assert np.isfinite(rows[:n - 2 - n // 2][s[:n - 2 - n // 2] < 0]).all()
     assert (rows[-2:, :, 7][s[-2:] < 0] == -np.inf).all()
+
+
+def test_attn_prefill_two_threads_one_stream(gpu):
+    """Two host threads with prompts of their own, and of growing lengths, on the null stream: every call gives the bytes it
+    gives alone."""
+    torch = gpu
+    nh, nkv, sizes = 32, 8, (650, 700, 900, 1200)
+    jobs = []
+    for t in range(2):
+        rng = np.random.default_rng(t)
+        q = torch.from_numpy(rng.standard_normal((sizes[-1], nh * 128)).astype(np.float32)).cuda()
+        kv = torch.from_numpy(rng.standard_normal((2, nkv, sizes[-1], 128)).astype(np.float32)).cuda()
+        jobs.append((q, kv, [torch.empty(n, nh, 128, device="cuda") for n in sizes for _ in range(8)]))
+
+    def call(q, kv, n, out):
+        A.check(A.lib().aeth_attn_prefill(q.data_ptr(), nh * 128, kv.data_ptr(), n, nh, nkv, 128, sizes[-1], out.data_ptr(),
+                                          None), "attn_prefill")
+
+    torch.cuda.synchronize()
+    start, errors = threading.Barrier(2), []
+
+    def work(q, kv, outs):
+        try:
+            start.wait()
+            for out in outs:
+                call(q, kv, out.shape[0], out)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=j) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    for q, kv, outs in jobs:
+        for out in outs:
+            alone = torch.empty_like(out)
+            call(q, kv, out.shape[0], alone)
+            torch.cuda.synchronize()
+            assert torch.equal(out, alone)
 
 
 # ── device LlamaRunner vs the oracle's decode step ───────────────────────
