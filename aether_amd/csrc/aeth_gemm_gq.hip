@@ -463,11 +463,19 @@ bool aeth_gq_gemm_rows(const aeth_weight* w, int64_t m) {
     if (w->n % 256 != 0 || w->k < 4 || w->k > 65536 || w->n > (1LL << 28) || m > (1LL << 20)) return false;
     // grids below 2^32 threads (a larger product goes on as blocks that straddle inputs do)
     if (aeth_cdiv(m, 64) * (w->n / 256) > (1LL << 22) || w->n / 256 * aeth_cdiv(w->k, GQ_KS) > (1LL << 23)) return false;
-    // k_colk reads the weight once per 8 rows; this product costs about the same up to 64. At 8 / 16 / 24 rows, here
-    // against there: Q3_K 4096 × 4096 35 / 37 / 36 µs and 21 / 28 / 36, 14336 × 4096 (from 40 million weights on)
-    // 55 / 57 / 59 and 39 / 64 / 85; Q2_K 4096 × 4096 - / 42 / 40 and - / 29 / 38, 14336 × 4096 at 16 rows 74 and 68.
-    if (w->n * w->k >= 40000000) return m > (w->dtype == AETH_DTYPE_Q2_K ? 16 : 8);
-    return m > 24;
+    // From the rows that had the f64 product, always (its precision). Below: k_colk goes through the weight once per 8
+    // rows, g times, here it is unpacked and read whole, plus a fixed ≈ 20 µs of launches; both times grow with the weight,
+    // in M = 10^6 weights ≈ 0.45·g·M + 8 there and 0.62·M + 20 here (Q2_K: 1.0·M + 24, the mins' product too). So from
+    // (g − 1.3)·M = 23 on (Q2_K: (g − 1.95)·M = 26). µs here / there, last row count there and first here:
+    // Q3_K 4096 × 2048 (8.4) 24 rows 28.8 / 25.6, 32 29.4 / 27.9; 4096 × 4096 (16.8) 16 36.3 / 26.7, 24 34.6 / 35.2; 6144 ×
+    // 4096 (25) 16 36.3 / 36.4, 24 36.0 / 45.6; 2048 × 14336 (29) 16 42.5 / 36.9, 24 41.8 / 47.2; 8192 × 4096 (34) 8 38.7 /
+    // 27.7, 16 37.4 / 42.3; 4096 × 14336 (59) 8 54.6 / 35.5, 16 56.0 / 59.1; 28672 × 4096 (117) 8 93 / 65, 16 95 / 122.
+    // Q2_K 4096 × 4096 24 39.6 / 36.8, 32 37.7 / 42.8; 6144 × 4096 16 45.9 / 37.0, 24 45.7 / 48.2; 14336 × 2048 16 49.8 / 42.5,
+    // 24 50.5 / 52.2; 14336 × 4096 16 75.9 / 67.4, 24 78.2 / 88.7; 28672 × 4096 16 134 / 128, 24 137 / 164.
+    const bool q2 = w->dtype == AETH_DTYPE_Q2_K;
+    const int64_t g = aeth_cdiv(m, 8), weights = w->n * w->k;
+    if (m >= (q2 ? 40 : 32)) return true;
+    return q2 ? (20 * g - 39) * weights >= 520000000 : (10 * g - 13) * weights >= 230000000;
 }
 
 // bytes of the four unpacked arrays, rounded to 256

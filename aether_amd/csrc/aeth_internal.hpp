@@ -172,7 +172,7 @@ bool aeth_f16_gemm_rows(const aeth_weight* w, int64_t m);
 int aeth_gemm_f16_launch(const aeth_weight* w, const float* d_a, int64_t m, float* d_c, unsigned flags, hipStream_t s,
                          int64_t ldc = 0);
 // Whether m activation rows against GGUF-order Q2_K / Q3_K weight w take the int8 GEMM (aeth_gemm_gq.hip):
-// whole blocks per input (n % 256 == 0), k at most 65536, more than 24 rows (8 or 16 of a large weight).
+// whole blocks per input (n % 256 == 0), k at most 65536, from 9 (Q2_K 17) rows of a large weight to 32 (40) of any.
 bool aeth_gq_gemm_rows(const aeth_weight* w, int64_t m);
 int aeth_gemm_gq_launch(const aeth_weight* w, const float* d_a, int64_t m, float* d_c, unsigned flags, hipStream_t s,
                         int64_t ldc = 0);

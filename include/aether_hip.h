@@ -131,8 +131,9 @@ AETH_API int aeth_load_quant(int dtype, const void* d_src, int64_t k, int64_t n,
  *     below that; Q5_K / Q6_K / Q8_0 products the GEMMs do not take (k not
  *     whole super-blocks / blocks, buffers past 32-bit offsets) run the
  *     row-batched GEMV up to 80 / 80 / 112 rows, then the DGEMM below;
- *   - m > 1, GGUF-order Q2_K / Q3_K: the row-batched kernel up to 24 rows (Q3_K 8,
- *     Q2_K 16 from 40 million weights on), then the int8 MFMA product; with n not
+ *   - m > 1, GGUF-order Q2_K / Q3_K: the row-batched kernel for few rows (Q3_K up
+ *     to 8 of the largest weights, 31 of the smallest; Q2_K 16 and 39), then the
+ *     int8 MFMA product; with n not
  *     a multiple of 256 (blocks straddling inputs) up to a per-format row count
  *     (Q2_K 40, Q3_K 32), then the weight dequantized once and one rocBLAS f64
  *     DGEMM (also every K-quant product of the dot-product mode with k not a

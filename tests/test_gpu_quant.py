@@ -898,7 +898,7 @@ def test_gguf_packed_kernel_edges(gpu, dtype, m, n, k):
 
 @pytest.mark.parametrize("dtype", [Q2_K, Q3_K])
 @pytest.mark.parametrize("m,n,k", [(25, 256, 64), (33, 512, 100), (64, 256, 37), (65, 768, 1001), (130, 256, 4100),
-                                   (300, 2048, 320), (17, 10240, 4096)])
+                                   (300, 2048, 320), (17, 10240, 4096), (40, 256, 64), (47, 512, 100), (17, 6144, 4352)])
 def test_gguf_int8_gemm_edges(gpu, dtype, m, n, k):
     """The int8 product of GGUF-order Q2_K / Q3_K batches at row-tile, step and K-split remainders, uniformly random
     block bytes (scales of every exponent and sign), rows scaled 2^30 and 2^-30 and a zero row, A off 16-byte
@@ -948,7 +948,7 @@ FAR = [{5: 1e3}, {17: 1e4}, {300: 1e5}, {511: 1e6}, {0: 1e8}, {64: 1e30}, {3: -1
 
 
 @pytest.mark.parametrize("dtype", [Q2_K, Q3_K])
-@pytest.mark.parametrize("m,n,k,scales", [(33, 512, 1100, False), (70, 256, 4096, False), (40, 768, 640, True),
+@pytest.mark.parametrize("m,n,k,scales", [(41, 512, 1100, False), (70, 256, 4096, False), (40, 768, 640, True),
                                             (40, 768, 320, False)])
 def test_gguf_int8_gemm_far_values(gpu, dtype, m, n, k, scales):
     """One activation or block scale 10^3 .. 10^33 times the others of its row, whose integer weights are 0 in every other
@@ -1050,7 +1050,7 @@ def test_gemm_f16_tiles_scales_infinities(gpu, m, n, k):
 
 
 # a smaller batch of a larger weight leaves the row-batched kernel enough scratch, the GEMMs' own was never allocated
-@pytest.mark.parametrize("dtype,warm,m,n,k", [(Q3_K, (24, 8192), 25, 4096, 1024), (Q2_K, (24, 8192), 28, 4096, 1024),
+@pytest.mark.parametrize("dtype,warm,m,n,k", [(Q3_K, (8, 65536), 15, 16384, 2048), (Q2_K, (8, 65536), 17, 12288, 2048),
                                               (F16, (8, 12288), 32, 4096, 1024)])
 def test_batch_under_capture_without_gemm_scratch(gpu, dtype, warm, m, n, k):
     """Under graph capture no scratch can grow: a batch whose GEMM would need one takes the row-batched kernel when
