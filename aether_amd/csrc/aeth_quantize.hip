@@ -15,6 +15,7 @@
 // operand like fmaxf / fminf, and `as u8 / as i8` after the clamps is exact. The f16 scale bytes follow half::f16::from_f32:
 // round-to-nearest-even, NaN keeps its sign and top payload bits with the
 // quiet bit set.
+#include <algorithm>
 #include <type_traits>
 
 #include "aeth_common.hpp"
@@ -251,16 +252,17 @@ __device__ __forceinline__ void rq_part(const float (&v)[64], int p, int slot, i
     }
 }
 
-// f32 rows → blocks: a workgroup takes 64 consecutive super-blocks, staged through LDS so that
+// f32 rows → blocks: a workgroup takes SLOTS consecutive super-blocks, staged through LDS so that
 // a wave's loads are contiguous and part p of 64 super-blocks is one conflict-free column read.
-// A row's last super-block may be partial (RAGGED): its missing elements read as 0.
-template <int F, bool RAGGED>
+// A row's last super-block may be partial (RAGGED): its missing elements read as 0. With 16 slots
+// the threads past 4 · 16 form the same parts again (the same values to the same places).
+template <int F, bool RAGGED, int SLOTS>
 __global__ void __launch_bounds__(256) k_requant(const float* __restrict__ src, int64_t rows, int64_t cols, int64_t sbr,
                                                  int64_t row_bytes, uint8_t* __restrict__ out) {
-    constexpr int SLOTS = 64, XS = 257, OSD = Rq<F>::OSD;
+    constexpr int XS = 257, OSD = Rq<F>::OSD;
     __shared__ __attribute__((aligned(16))) uint32_t buf[SLOTS * XS];
     __shared__ RqShared<SLOTS> sh;
-    const int tid = threadIdx.x, slot = tid & 63, p = tid >> 6;
+    const int tid = threadIdx.x, slot = tid % SLOTS, p = tid / SLOTS & 3;
     const int64_t b0 = (int64_t)blockIdx.x * SLOTS, total = rows * sbr;
     float* x = (float*)buf;
 #pragma unroll 8
@@ -465,24 +467,39 @@ __global__ void __launch_bounds__(256) k_transpose_f32(const float* __restrict__
 }
 
 template <int F>
-static void requant_go(const float* src, int64_t rows, int64_t cols, uint8_t* dst, unsigned grid, hipStream_t s) {
-    const int64_t sbr = aeth_cdiv(cols, 256);
+static void requant_go(const float* src, int64_t rows, int64_t cols, uint8_t* dst, hipStream_t s) {
+    const int64_t sbr = aeth_cdiv(cols, 256), n = rows * sbr;
     const int64_t row_bytes = F == AETH_DTYPE_Q8_0 ? aeth_cdiv(cols, 32) * Q8_BLOCK_BYTES : sbr * Rq<F>::BB;
-    if (cols % 256 == 0)
-        hipLaunchKernelGGL((k_requant<F, false>), dim3(grid), dim3(256), 0, s, src, rows, cols, sbr, row_bytes, dst);
-    else
-        hipLaunchKernelGGL((k_requant<F, true>), dim3(grid), dim3(256), 0, s, src, rows, cols, sbr, row_bytes, dst);
+    // 16 super-blocks a workgroup (64 left most CUs idle up to 16384 of them, and put two a CU by their LDS after that): Q8_0
+    // 16 × 4096 21.6 → 8.1 µs, 1024 × 4096 24.7 → 16.2, 14336 × 4096 291 → 170; Q4_K 19 → 7.9, 21.4 → 16.0, 209 → 156, between
+    // (2048 rows) 25.9 → 28.0. The 64 stay for many ragged rows of Q4_K / Q5_K, where each super-block is mostly VALU
+    // work for absent elements: Q4_K 4096 × 300 24.9 → 15.0, but 32768 × 50 27.9 → 41.3, 65536 × 300 143 → 170.
+    constexpr bool wide = F == AETH_DTYPE_Q4_K || F == AETH_DTYPE_Q5_K;
+    const int64_t step = std::max<int64_t>(1, (1LL << 27) / sbr);  // rows a launch: below 2^32 threads
+    for (int64_t r = 0; r < rows; r += step) {
+        const float* x = src + r * cols;
+        uint8_t* o = dst + r * row_bytes;
+        const int64_t m = std::min(step, rows - r);
+        const dim3 grid((unsigned)aeth_cdiv(m * sbr, 16)), grid64((unsigned)aeth_cdiv(m * sbr, 64));
+        if (cols % 256 == 0)
+            hipLaunchKernelGGL((k_requant<F, false, 16>), grid, dim3(256), 0, s, x, m, cols, sbr, row_bytes, o);
+        else if (!wide || n < 64LL * aeth_num_cus())
+            hipLaunchKernelGGL((k_requant<F, true, 16>), grid, dim3(256), 0, s, x, m, cols, sbr, row_bytes, o);
+        else if constexpr (wide)
+            hipLaunchKernelGGL((k_requant<F, true, 64>), grid64, dim3(256), 0, s, x, m, cols, sbr, row_bytes, o);
+    }
 }
 
 static int requant_launch(int dtype, const float* src, int64_t rows, int64_t cols, uint8_t* dst, hipStream_t s) {
-    const int64_t groups = aeth_cdiv(rows * aeth_cdiv(cols, 256), 64);
-    if (groups == 0) return AETH_OK;
-    if (groups > 0x7FFFFFFF) return aeth_set_error(AETH_EINVAL, "requantize: too many blocks");
-    const unsigned grid = (unsigned)groups;
-    if (dtype == AETH_DTYPE_Q8_0) requant_go<AETH_DTYPE_Q8_0>(src, rows, cols, dst, grid, s);
-    else if (dtype == AETH_DTYPE_Q4_K) requant_go<AETH_DTYPE_Q4_K>(src, rows, cols, dst, grid, s);
-    else if (dtype == AETH_DTYPE_Q5_K) requant_go<AETH_DTYPE_Q5_K>(src, rows, cols, dst, grid, s);
-    else requant_go<AETH_DTYPE_Q6_K>(src, rows, cols, dst, grid, s);
+    if (dtype == AETH_DTYPE_Q8_0 && cols % 32 == 0) {  // whole blocks a row: one run of blocks, no row's end to pad
+        cols *= rows;
+        rows = 1;
+    }
+    if (rows == 0 || cols == 0) return AETH_OK;
+    if (dtype == AETH_DTYPE_Q8_0) requant_go<AETH_DTYPE_Q8_0>(src, rows, cols, dst, s);
+    else if (dtype == AETH_DTYPE_Q4_K) requant_go<AETH_DTYPE_Q4_K>(src, rows, cols, dst, s);
+    else if (dtype == AETH_DTYPE_Q5_K) requant_go<AETH_DTYPE_Q5_K>(src, rows, cols, dst, s);
+    else requant_go<AETH_DTYPE_Q6_K>(src, rows, cols, dst, s);
     AETH_LAUNCH_CHECK();
     return AETH_OK;
 }

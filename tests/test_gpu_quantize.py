@@ -65,6 +65,23 @@ def test_requantize_byte_exact(gpu, dtype, rows, cols):
         dtype, bad.size, got.size, bad[0], bad[0] // bb, got[bad[0]], ref[bad[0]])
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,cols", [(1, 256), (17, 256), (5, 96), (300, 32), (7, 224), (33, 40), (3, 5000), (16400, 33)])
+def test_requantize_workgroups(gpu, dtype, rows, cols):
+    """16 super-blocks a workgroup with part-filled last ones, Q8_0 rows of whole blocks as one run of blocks (a short last
+    super-block), and the 64 of many ragged Q4_K / Q5_K rows (16400 of them): every byte, and none past the last."""
+    torch = gpu
+    x = special_rows(np.random.default_rng(rows + cols + dtype), rows, cols)
+    be, bb = GEOM[dtype]
+    nbytes = rows * ((cols + be - 1) // be) * bb
+    out = torch.full((nbytes + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+    xd = to_dev(torch, x)
+    A.check(A.lib().aeth_requantize(dtype, xd.data_ptr(), rows, cols, out.data_ptr(), None), "requantize")
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:nbytes], O.requantize(dtype, x.ravel(), rows, cols)) and (got[nbytes:] == 0xA5).all()
+
+
 @pytest.mark.parametrize("m,k", [(1, 32), (3, 100), (8, 4096), (9, 1000), (2, 31)])
 def test_quantize_activations_q8_0_byte_exact(gpu, m, k):
     torch = gpu
