@@ -101,6 +101,10 @@ WIDTHS = {
     # epilogue (k_gemm_tail_sum writes h); the down GEMM's plain prep reads k = 16640 in two register chunks
     "d4096_ff16640": (dict(vocab_size=4096, d_model=4096, num_layers=1, num_heads=32, num_kv_heads=8, d_ff=16640),
                       "2 / plain, 33 steps (8 8 8 9) in two chunks"),
+    # the gate|up GEMM's 2 × 384 = 768 tiles of 64 × 128 are 192 of 128 × 256, three rounds of 256 CUs for one: it runs
+    # k_gemm_q4k_big with the RMSNorm in its prep and its SwiGLU epilogue, the last 58 of each tile's 128 rows empty
+    "d512_ff24576": (dict(vocab_size=4096, d_model=512, num_layers=1, num_heads=4, num_kv_heads=2, d_ff=24576),
+                     "1 / plain, 48 steps in two chunks"),
     "d2048_ff5632": (dict(vocab_size=4096, d_model=2048, num_layers=1, num_heads=16, num_kv_heads=4, d_ff=5632),
                      "1 / 4 (11 steps: 2 3 3 3)"),
 }
@@ -111,9 +115,10 @@ def test_prefill_8b_widths_match_oracle(gpu, width):
     """Batched prefill (forward_batch, runner.rs:833-993) of 70 tokens: the
     Q4_K GEMMs with the RMSNorm (q|k|v, gate|up at k = d_model) and the
     SwiGLU (down, k = d_ff) run inside their activation prep; 70 rows leave
-    58 rows of the last 64-row tile empty. The 8B widths and four others
+    58 rows of the last 64-row tile empty. The 8B widths and five others
     that reach the prep's other register shares (and, at d_ff 16640, the
-    gate|up GEMM's last-round K split under its SwiGLU epilogue)."""
+    gate|up GEMM's last-round K split, at d_ff 24576 its 128 × 256 tiles
+    under its SwiGLU epilogue)."""
     c = dict(C8B, max_seq_len=256, **WIDTHS[width][0])
     L = A.lib()
     d, dff, V = c["d_model"], c["d_ff"], c["vocab_size"]
