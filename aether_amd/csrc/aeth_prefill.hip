@@ -497,14 +497,21 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill_mf(const float* __restr
 //    maximum that may be 2^8 stale, and a tile's enter its product times a power
 //    of two of their column's largest, so that neither a flat row nor a tile far
 //    below the maximum has them in fp16's subnormals.
-// What bounds it: at n = 2000 (32 / 8 heads: 325 → 126 µs, 8 of it k_attn_split) the matrix cores are busy a third
+// What bounds it: at n = 2000 (32 / 8 heads: 325 → 117 µs, 7 of it k_attn_split) the matrix cores are busy a third
 // of the time, 30 % of the waves' time goes to waits for LDS and the stage barrier, 37 % to dependencies. Not the
 // phases of a SIMD's two waves: an odd wave that multiplies its values a stage late took 138 µs, four
 // independent chains in place of two 153; without the stage loads it would take 115.
-// A KV head with an infinity or NaN among its keys or values takes a plain f32
-// loop (the split has no infinities).
+// The parts are 22 bits of a value while it is no smaller than 2^-16 of the largest that shares its power of two (below
+// that a fixed 2^-39 of the largest). Where that would show, f32 sums on the VALU run instead (sp_plain, 880 .. 980 µs for
+// that prompt): for a KV head of which some tile has SP_FEW groups of eight (eight dimensions of a key; a dimension of eight
+// values' rows) below 2^-16 of its largest and not all zero, so that a key or a dimension is out of proportion (a key has 16
+// such groups, a dimension of the values 4; of normal numbers a group with one key left in the last tile is one in 10^4
+// times), or an infinity or NaN (the split has none, and a masked key's must not reach the queries before it); and for
+// 128 columns with a query of which, of a lane's eight groups of eight dimensions, five stay below 2^-13 of its largest.
 #define SP_TILE 32768  // bytes of a key tile's fragments: K [8 k-steps][hi, lo][1 KiB], V [4 d-tiles][2 halves][hi, lo][1 KiB]
-#define SP_BAD 0x7FFF  // exponent of a tile holding an infinity or NaN
+#define SP_BAD 0x7FFF  // exponent of a tile for sp_plain: an infinity or NaN, too wide a range, or numbers past 2^64
+#define SP_MAXE 50     // largest exponent of a score's factors: no product of their scales overflows
+#define SP_FEW 4       // groups of eight numbers below 2^-16 of the largest that make a tile's range too wide
 
 typedef _Float16 sp_h8 __attribute__((ext_vector_type(8)));
 typedef float sp_f16 __attribute__((ext_vector_type(16)));
@@ -525,18 +532,21 @@ __device__ __forceinline__ int sp_exponent(float mx) {
     return max(E - 14, -100);
 }
 
+// a group's largest number g below 2^-bits of the largest mx, and not zero
+__device__ __forceinline__ bool sp_small(float g, float mx, int bits) { return g > 0.0f && g < ldexpf(mx, -bits); }
+
 __global__ void __launch_bounds__(256) k_attn_split(const float* __restrict__ layer_kv, int n, int nkv, int64_t max_seq,
                                                     int ntiles, uint8_t* __restrict__ frag, int2* __restrict__ exps) {
     __shared__ float red[2][4];
-    __shared__ int bad;
+    __shared__ int bad, few;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int g = blockIdx.x % nkv, t = blockIdx.x / nkv, k0 = 32 * t;
     const float* K = layer_kv + (int64_t)g * max_seq * 128;
     const float* V = layer_kv + (int64_t)(nkv + g) * max_seq * 128;
-    if (tid == 0) bad = 0;
+    if (tid == 0) bad = few = 0;
     // K: k-steps w and w + 4, lane = key lane%32, d 16·ks + 8·(lane/32) + i. V: (d-tile, half) pairs w and w + 4,
     // lane = d 32·dt + lane%32, element i = key 16·half + 8·(i/4) + 4·(lane/32) + i%4 (Sᵀ's result order)
-    float kx[2][8], vx[2][8], km = 0.0f, vm = 0.0f;
+    float kx[2][8], vx[2][8], km = 0.0f, vm = 0.0f, kg[2] = {}, vg[2] = {};
     bool nf = false;
 #pragma unroll
     for (int u = 0; u < 2; u++) {
@@ -552,10 +562,12 @@ __global__ void __launch_bounds__(256) k_attn_split(const float* __restrict__ la
             const float x = V[(int64_t)min(vk, n - 1) * 128 + 32 * dt + (lane & 31)];
             vx[u][i] = vk < n ? x : 0.0f;
             nf |= !(fabsf(kx[u][i]) < INFINITY) || !(fabsf(vx[u][i]) < INFINITY);
-            km = fmaxf(km, fabsf(kx[u][i]));
-            vm = fmaxf(vm, fabsf(vx[u][i]));
+            kg[u] = fmaxf(kg[u], fabsf(kx[u][i]));
+            vg[u] = fmaxf(vg[u], fabsf(vx[u][i]));
         }
     }
+    km = fmaxf(kg[0], kg[1]);
+    vm = fmaxf(vg[0], vg[1]);
     km = aeth_wave_max(km);
     vm = aeth_wave_max(vm);
     __syncthreads();
@@ -565,8 +577,11 @@ __global__ void __launch_bounds__(256) k_attn_split(const float* __restrict__ la
         red[1][w] = vm;
     }
     __syncthreads();
-    const int ek = sp_exponent(fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3])));
-    const int ev = sp_exponent(fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3])));
+    km = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+    vm = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
+    const int ek = sp_exponent(km), ev = sp_exponent(vm);
+    const int c = sp_small(kg[0], km, 16) + sp_small(kg[1], km, 16) + sp_small(vg[0], vm, 16) + sp_small(vg[1], vm, 16);
+    if (c) atomicAdd(&few, c);
     const float ki = ldexpf(1.0f, -ek), vi = ldexpf(1.0f, -ev);
     uint8_t* dst = frag + ((int64_t)g * ntiles + t) * SP_TILE + lane * 16;
 #pragma unroll
@@ -579,29 +594,131 @@ __global__ void __launch_bounds__(256) k_attn_split(const float* __restrict__ la
         *(sp_h8*)(dst + 16384 + (w + 4 * u) * 2048) = hi;
         *(sp_h8*)(dst + 16384 + (w + 4 * u) * 2048 + 1024) = lo;
     }
-    if (tid == 0) exps[g * ntiles + t] = bad ? make_int2(SP_BAD, SP_BAD) : make_int2(ek, ev);
+    __syncthreads();
+    if (tid == 0) {
+        const bool wide = few >= SP_FEW || ek > SP_MAXE || ev > SP_MAXE;
+        exps[g * ntiles + t] = bad || wide ? make_int2(SP_BAD, SP_BAD) : make_int2(ek, ev);
+    }
 }
 
-// Rows of a KV head with an infinity or NaN in its cache: thread = (column tid/4, d [32·(tid%4), +32)), plain f32.
+// 128 columns in f32 on the VALU (rare), the queries from q0 on: tiles of 32 keys through LDS, thread = (two columns
+// 2·(tid/8), dimensions [16·(tid%8), +16)), a score summed over eight lanes. A masked key's value enters nothing.
+struct SpPlain {
+    float k[32][132], v[32][132], p[128][33];
+};
 template <int G>
-__device__ __noinline__ void sp_plain(const float* qkv, int64_t qkv_stride, const float* K, const float* V, int n, int nh,
-                                      int g, int q0, int window, float* out) {
-    const int cc = threadIdx.x >> 2, d0 = 32 * (threadIdx.x & 3), query = q0 + cc / G, head = g * G + cc % G;
-    if (query >= n) return;
-    const float* q = qkv + (int64_t)query * qkv_stride + (int64_t)head * 128;
+__device__ __forceinline__ void sp_plain(const float* qkv, int64_t qkv_stride, const float* K, const float* V, int n, int nh,
+                                      int g, int q0, int window, float* out, SpPlain* sh) {
+    const int tid = threadIdx.x, c0 = 2 * (tid >> 3), part = tid & 7, d0 = 16 * part;
     const float scale = 1.0f / sqrtf(128.0f);
-    float m = -INFINITY, l = 0.0f, o[32] = {};
-    for (int t = window > 0 ? max(0, query - window + 1) : 0; t <= query; t++) {
-        float s = 0.0f;
-        for (int d = 0; d < 128; d++) s = fmaf(q[d], K[(int64_t)t * 128 + d], s);
-        s *= scale;
-        const float mn = fmaxf(m, s), al = mn == -INFINITY ? 1.0f : expf(m - mn);
-        const float p = mn == -INFINITY ? 0.0f : expf(s - mn);
-        l = l * al + p;
-        for (int d = 0; d < 32; d++) o[d] = o[d] * al + p * V[(int64_t)t * 128 + d0 + d];
-        m = mn;
+    int query[2], lo[2];  // keys [lo, query] are visible
+    float q[2][16], o[2][16] = {}, m[2] = {-INFINITY, -INFINITY}, l[2] = {};
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        query[c] = q0 + (c0 + c) / G;
+        lo[c] = window > 0 ? query[c] - window + 1 : 0;
+        const float* src = qkv + (int64_t)min(query[c], n - 1) * qkv_stride + (int64_t)(g * G + (c0 + c) % G) * 128 + d0;
+#pragma unroll
+        for (int d = 0; d < 16; d += 4) {
+            const float4 x = *(const float4*)(src + d);
+            q[c][d] = x.x; q[c][d + 1] = x.y; q[c][d + 2] = x.z; q[c][d + 3] = x.w;
+        }
     }
-    for (int d = 0; d < 32; d++) out[(int64_t)query * nh * 128 + (int64_t)head * 128 + d0 + d] = o[d] * (1.0f / l);
+    const int kb_end = (min(q0 + 128 / G, n) - 1) / 32, kb_beg = window > 0 ? max(0, q0 - window + 1) / 32 : 0;
+    for (int kb = kb_beg; kb <= kb_end; kb++) {
+        __syncthreads();
+        for (int i = tid; i < 32 * 32; i += 512) {
+            const int t = i >> 5, d = 4 * (i & 31);
+            *(float4*)&sh->k[t][d] = *(const float4*)(K + (int64_t)min(32 * kb + t, n - 1) * 128 + d);
+            *(float4*)&sh->v[t][d] = *(const float4*)(V + (int64_t)min(32 * kb + t, n - 1) * 128 + d);
+        }
+        __syncthreads();
+        float s[2][4], mx[2] = {-INFINITY, -INFINITY};  // of this lane's keys part + 8u
+#pragma unroll
+        for (int t = 0; t < 32; t++) {
+            float a[2] = {0.0f, 0.0f};
+#pragma unroll
+            for (int d = 0; d < 16; d += 4) {
+                const float4 y = *(const float4*)&sh->k[t][d0 + d];
+#pragma unroll
+                for (int c = 0; c < 2; c++) {
+                    a[c] = fmaf(q[c][d], y.x, a[c]);
+                    a[c] = fmaf(q[c][d + 1], y.y, a[c]);
+                    a[c] = fmaf(q[c][d + 2], y.z, a[c]);
+                    a[c] = fmaf(q[c][d + 3], y.w, a[c]);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                a[c] += aeth_dpp_xor1f(a[c]);
+                a[c] += aeth_dpp_xor2f(a[c]);
+                a[c] += aeth_dpp_mirror8f(a[c]);
+                s[c][t >> 3] = (t & 7) == part ? a[c] * scale : s[c][t >> 3];
+            }
+            if ((t & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // four keys' reads in flight
+        }
+        float al[2];
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int t = 32 * kb + part + 8 * u;
+                if (t < lo[c] || t > query[c]) s[c][u] = -INFINITY;
+                mx[c] = fmaxf(mx[c], s[c][u]);
+            }
+            mx[c] = fmaxf(mx[c], aeth_dpp_xor1f(mx[c]));
+            mx[c] = fmaxf(mx[c], aeth_dpp_xor2f(mx[c]));
+            mx[c] = fmaxf(mx[c], aeth_dpp_mirror8f(mx[c]));
+            const float mn = fmaxf(m[c], mx[c]);
+            al[c] = mn == -INFINITY ? 1.0f : expf(m[c] - mn);
+            m[c] = mn;
+            l[c] *= al[c];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int t = 32 * kb + part + 8 * u;
+                const float p = t >= lo[c] && t <= query[c] && mn != -INFINITY ? expf(s[c][u] - mn) : 0.0f;
+                sh->p[c0 + c][part + 8 * u] = p;
+                l[c] += p;
+            }
+#pragma unroll
+            for (int d = 0; d < 16; d++) o[c][d] *= al[c];
+        }
+        __syncthreads();
+        const int t0 = max(min(lo[0], lo[1]) - 32 * kb, 0), t1 = min(max(query[0], query[1]) - 32 * kb, 31);
+#pragma unroll 4
+        for (int t = t0; t <= t1; t++) {
+            float4 y[4];
+#pragma unroll
+            for (int d = 0; d < 4; d++) y[d] = *(const float4*)&sh->v[t][d0 + 4 * d];
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const int key = 32 * kb + t;
+                const float p = sh->p[c0 + c][t];
+                if (key < lo[c] || key > query[c]) continue;
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    o[c][4 * d] = fmaf(p, y[d].x, o[c][4 * d]);
+                    o[c][4 * d + 1] = fmaf(p, y[d].y, o[c][4 * d + 1]);
+                    o[c][4 * d + 2] = fmaf(p, y[d].z, o[c][4 * d + 2]);
+                    o[c][4 * d + 3] = fmaf(p, y[d].w, o[c][4 * d + 3]);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        l[c] += aeth_dpp_xor1f(l[c]);
+        l[c] += aeth_dpp_xor2f(l[c]);
+        l[c] += aeth_dpp_mirror8f(l[c]);
+        const float inv = 1.0f / l[c];
+        if (query[c] < n) {
+            float* dst = out + (int64_t)query[c] * nh * 128 + (int64_t)(g * G + (c0 + c) % G) * 128 + d0;
+#pragma unroll
+            for (int d = 0; d < 16; d += 4)
+                *(float4*)(dst + d) = make_float4(o[c][d] * inv, o[c][d + 1] * inv, o[c][d + 2] * inv, o[c][d + 3] * inv);
+        }
+    }
+    __syncthreads();  // LDS is used again
 }
 
 template <int G>
@@ -615,8 +732,10 @@ __global__ void __launch_bounds__(512, 2) k_attn_prefill_sp(const float* __restr
     constexpr float TH = 8.0f;  // log2: how stale a maximum may be
     // two stages of two tiles (128 KiB), then the partial results [key parity][column][PLD] and their statistics
     __shared__ __attribute__((aligned(1024))) char smem[2 * 128 * PLD * 4];
+    static_assert(sizeof(SpPlain) <= sizeof(smem), "the f32 form's LDS");
     __shared__ float pm[2][128], pl[2][128];
     __shared__ int pe[2][4];
+    __shared__ __attribute__((aligned(16))) int far[2][8];  // [pass][wave]: a query of the wave's is for sp_plain
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), cg = w & 3, par = w >> 2;
     const int c = 32 * cg + (lane & 31), hf = lane >> 5;
@@ -628,17 +747,20 @@ __global__ void __launch_bounds__(512, 2) k_attn_prefill_sp(const float* __restr
     bool bad = false;
     for (int t = lane; t < ntiles; t += 64) bad |= ex[t].x == SP_BAD;
     bad = __any(bad);
+    if (lane < 2) far[lane][w] = 0;  // (a wave's own: no barrier; a store to LDS under the stage's loads would wait for them)
+    if (lane < 2) far[lane][w] = 0;  // (a wave's own: no barrier; a store to LDS under the stage's loads would wait for them)
+    auto plain = [&](int q0) {
+        sp_plain<G>(qkv, qkv_stride, layer_kv + (int64_t)g * max_seq * 128, layer_kv + (int64_t)(nkv + g) * max_seq * 128, n, nh,
+                    g, q0, window, out, (SpPlain*)smem);
+    };
     const uint32_t sm0 = lds_addr(smem);
     const float sl2 = 1.4426950408889634f / sqrtf(128.0f);  // scale · log2(e)
     for (int pass = 0; pass < 2; pass++) {
         const int qb = pass == 0 ? p : nqb - 1 - p;
         if (pass == 1 && qb == p) break;  // the middle block of an odd count (uniform)
         const int q0 = qb * QB, query = q0 + c / G;
-        if (bad) {
-            sp_plain<G>(qkv, qkv_stride, layer_kv + (int64_t)g * max_seq * 128,
-                        layer_kv + (int64_t)(nkv + g) * max_seq * 128, n, nh, g, q0, window, out);
-            continue;
-        }
+        bool again = bad;
+        if (!bad) {
         const int kb_end = (min(q0 + QB, n) - 1) / 32;                           // last key tile, inclusive
         const int kb_beg = window > 0 ? max(0, q0 - window + 1) / 32 : 0;        // first one any query sees
         const int w_lo = q0 + 32 * cg / G, w_hi = q0 + (32 * cg + 31) / G;       // this wave's queries
@@ -654,17 +776,23 @@ __global__ void __launch_bounds__(512, 2) k_attn_prefill_sp(const float* __restr
         float fq;
         {
             const float* src = qkv + (int64_t)min(query, n - 1) * qkv_stride + (int64_t)head * 128 + 8 * hf;
-            float x[8][8], mx = 0.0f;
+            float x[8][8], xg[8], mx = 0.0f;
 #pragma unroll
             for (int ks = 0; ks < 8; ks++) {
                 const float4 a = *(const float4*)(src + 16 * ks), b = *(const float4*)(src + 16 * ks + 4);
                 x[ks][0] = a.x; x[ks][1] = a.y; x[ks][2] = a.z; x[ks][3] = a.w;
                 x[ks][4] = b.x; x[ks][5] = b.y; x[ks][6] = b.z; x[ks][7] = b.w;
 #pragma unroll
-                for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(x[ks][i]));
+                for (int i = 0; i < 8; i++) xg[ks] = i ? fmaxf(xg[ks], fabsf(x[ks][i])) : fabsf(x[ks][0]);
+                mx = fmaxf(mx, xg[ks]);
             }
             mx = pa_max32(mx);
             const int eq = sp_exponent(mx < INFINITY ? mx : 0.0f);  // an infinity makes the column NaN
+            int few = eq > SP_MAXE ? 8 : 0;
+#pragma unroll
+            for (int ks = 0; ks < 8; ks++) few += sp_small(xg[ks], mx, 13) ? 1 : 0;
+            if (__any(few > 4)) far[pass][w] = 1;  // (a branch: the store waits for the loads in flight) read after the pass
+            __builtin_amdgcn_sched_barrier(0);
             const float inv = ldexpf(1.0f, -eq);
 #pragma unroll
             for (int ks = 0; ks < 8; ks++) sp_split(x[ks], inv, qh[ks], ql[ks]);
@@ -829,12 +957,20 @@ __global__ void __launch_bounds__(512, 2) k_attn_prefill_sp(const float* __restr
             }
         }
         __syncthreads();  // LDS is reused by the second query block
+        const int4 f0 = *(const int4*)&far[pass][0], f1 = *(const int4*)&far[pass][4];
+        if (__builtin_amdgcn_readfirstlane(f0.x | f0.y | f0.z | f0.w | f1.x | f1.y | f1.z | f1.w)) again = true;
+        }
+        if (again)  // the pass's rows in f32
+            sp_plain<G>(qkv, qkv_stride, layer_kv + (int64_t)g * max_seq * 128, layer_kv + (int64_t)(nkv + g) * max_seq * 128, n,
+                        nh, g, q0, window, out, (SpPlain*)smem);
     }
 }
 
-// The split form where it is the faster one: its workgroups, one per pair of 128/G-query blocks and KV head, have to
-// fill enough of the chip. µs here and on the f32 kernel, 32 / 8 heads: n = 512 (64 workgroups) 41.6 / 37.3, 640 (80)
-// 48.0 / 59.6, 768 54 / 69.6, 1000 66 / 109, 2000 126 / 330, 4000 466 / 1318; 16 / 8 heads, n = 1000 (64) 62 / 57.
+// The split form where it is the faster one: once the f32 kernel's workgroups (eight for one of these) no longer fit the
+// chip at once, two a CU. µs here and on the f32 kernel by its workgroups on 256 CUs: 512 (32 / 8 heads, n = 512) 43.7 / 35.4,
+// (16 / 8, 1024) 63.3 / 51.4, (16 / 2, 1024) 62.6 / 51.9, (64 / 8, 256) 34.0 / 24.5; 544 (32 / 8, 544) 45.5 / 50.7, 576 46.7 / 51.2,
+// 552 (16 / 8, 1100) 68 / 79, 600 (32 / 4, 600) 48.8 / 52.7, 640 (64 / 8, 320) 37.0 / 37.4, (32 / 8, 640) 49 / 54; 1200 (32 / 4,
+// 1200) 74 / 136, n = 2000 at 32 / 8 heads 117 / 330, 4000 414 / 1318.
 // It needs a scratch of 32 KiB per KV head and 32 keys, the stream's own; under graph capture, where that could not grow
 // and a recorded address would not outlive a later growth, and where there is no memory for it, the f32 kernel runs.
 // Two host threads may call on one stream: from the fetch of the scratch to the launch that reads it a call holds a
@@ -845,7 +981,7 @@ static bool attn_split_launch(const float* qkv, int64_t stride, const float* lay
                               int64_t max_seq, int win, float* out, hipStream_t s, int* rc) {
     *rc = AETH_OK;
     const int64_t nqb = aeth_cdiv(n, 128 / G), wgs = nkv * aeth_cdiv(nqb, 2), nt = aeth_cdiv(n, 32);
-    if (wgs < 80) return false;
+    if (nkv * aeth_cdiv(aeth_cdiv(n, 16 / G), 2) <= 2 * aeth_num_cus()) return false;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
         (void)hipGetLastError();

@@ -235,10 +235,10 @@ def attn_prefill64(q, kv, n, nh, nkv, hd):
     return ref, mag, smax
 
 
-# enough rows that the fp16-split kernel takes them (80 pairs of 128/G-query blocks and KV heads): every group size,
+# enough rows that the fp16-split kernel takes them (the f32 kernel's workgroups past two a CU; 513 the first so): every group size,
 # odd and even block counts, a last key tile of 1 .. 32 keys; key tiles scaled 2^-2 .. 2^2 and value tiles 2^-12 ..
 # 2^12 against each other, so that the tiles' exponents differ
-@pytest.mark.parametrize("n,nh,nkv,max_seq", [(640, 32, 8, 640), (1025, 32, 8, 1100), (700, 64, 8, 704), (1300, 16, 8, 1300),
+@pytest.mark.parametrize("n,nh,nkv,max_seq", [(513, 32, 8, 520), (640, 32, 8, 640), (1025, 32, 8, 1100), (700, 64, 8, 704), (1300, 16, 8, 1300),
                                               (650, 32, 32, 1000)])
 def test_attn_prefill_split_matches_f64(gpu, n, nh, nkv, max_seq):
     """Error: a score is the f32 sum of 24 matrix-core steps over parts that leave 2^-22 of a product, at most 2^-19 of
@@ -323,6 +323,74 @@ def test_attn_prefill_two_threads_one_stream(gpu):
             call(q, kv, out.shape[0], alone)
             torch.cuda.synchronize()
             assert torch.equal(out, alone)
+
+
+def attn_prefill(torch, qd, stride, kvd, n, nh, nkv, max_seq, stream=None):
+    out = torch.full((n, nh, 128), float("nan"), device="cuda")
+    A.check(A.lib().aeth_attn_prefill(qd.data_ptr(), stride, kvd.data_ptr(), n, nh, nkv, 128, max_seq, out.data_ptr(),
+                                      stream), "attn_prefill")
+    return out
+
+
+# what the two fp16 parts of the split kernel cannot hold beside what shares their power of two: a key or a dimension of the
+# keys or values far above the others of its tile, one far below them, a dimension of some queries, and numbers whose
+# scales' product overflows
+WIDE = {"value": lambda q, k, v: v.__setitem__((0, 100), v[0, 100] * 1e9),
+        "value dim": lambda q, k, v: v.__setitem__((1, slice(640, 672), 5), v[1, 640:672, 5] * 1e8),
+        "small dim": lambda q, k, v: v.__setitem__((1, slice(0, None), 77), v[1, :, 77] * 1e-9),
+        "key": lambda q, k, v: (k.__setitem__((0, 300), k[0, 300] * 1e8), q.__setitem__((slice(0, None), slice(0, 128)), 0.0)),
+        "key dim": lambda q, k, v: (k.__setitem__((0, slice(0, None), 3), k[0, :, 3] * 1e9), q[:, 3:512:128].fill(0.0)),
+        "query dim": lambda q, k, v: (q[200:300, 9::128].__imul__(1e10), k.__setitem__((slice(0, None), slice(0, None), 9), 0.0)),
+        "scales": lambda q, k, v: (q[:, 9::128].__imul__(1e22), k.__setitem__((slice(0, None), 31, 9), 1e22),
+                                   k.__setitem__((slice(0, None), slice(0, 31), 9), 0.0))}
+
+
+@pytest.mark.parametrize("n,nh,nkv", [(700, 32, 8), (650, 64, 8)])
+@pytest.mark.parametrize("what", list(WIDE))
+def test_attn_prefill_wide_ranges(gpu, what, n, nh, nkv):
+    """Numbers that the fp16 parts would not hold take the f32 arithmetic: per output 2^-19·(2 + A)·Σ|p·v| (the bound of
+    the split kernel's test, here with nothing that grows with a number elsewhere in its tile)."""
+    torch = gpu
+    rng = np.random.default_rng(n)
+    stride = (nh + 2 * nkv) * 128
+    q = rng.standard_normal((n, stride)).astype(np.float32)
+    kv = rng.standard_normal((2, nkv, n, 128)).astype(np.float32)
+    WIDE[what](q, kv[0], kv[1])
+    ref, mag, smax = attn_prefill64(q, kv, n, nh, nkv, 128)
+    got = attn_prefill(torch, torch.from_numpy(q).cuda(), stride, torch.from_numpy(kv).cuda(), n, nh, nkv, n).cpu().numpy()
+    ok = np.isfinite(smax[..., 0]) & (smax[..., 0] < 1e30)
+    assert ok[:31].all()
+    assert (np.abs(got - ref)[ok] <= (2.0 ** -19 * (2 + smax) * mag)[ok] + 1e-44).all()
+
+
+def test_attn_prefill_under_capture(gpu):
+    """Under graph capture a long prompt runs the f32 kernel (its scratch could not grow): the same attention as outside it
+    to the bound of either, at every replay, with other eager work between the replays."""
+    torch = gpu
+    n, nh, nkv = 700, 32, 8
+    rng = np.random.default_rng(1)
+    stride = nh * 128
+    q, kv = torch.empty(n, stride, device="cuda"), torch.empty(2, nkv, n, 128, device="cuda")
+    out = torch.empty(n, nh, 128, device="cuda")
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        A.check(A.lib().aeth_attn_prefill(q.data_ptr(), stride, kv.data_ptr(), n, nh, nkv, 128, n, out.data_ptr(),
+                                          s.cuda_stream), "attn_prefill")
+    for _ in range(3):
+        qh = rng.standard_normal((n, stride)).astype(np.float32)
+        kvh = rng.standard_normal((2, nkv, n, 128)).astype(np.float32)
+        q.copy_(torch.from_numpy(qh))
+        kv.copy_(torch.from_numpy(kvh))
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        eager = attn_prefill(torch, q, stride, kv, n, nh, nkv, n).cpu().numpy()
+        ref, mag, smax = attn_prefill64(qh, kvh, n, nh, nkv, 128)
+        for got in (out.cpu().numpy(), eager):
+            assert (np.abs(got - ref) <= 2.0 ** -19 * (2 + smax) * mag).all()
 
 
 # ── device LlamaRunner vs the oracle's decode step ───────────────────────
