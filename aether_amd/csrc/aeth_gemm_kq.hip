@@ -212,8 +212,8 @@ __global__ void __launch_bounds__(64 * K8_W) k_gemm_kq(KqArgs G) {
 #pragma unroll
         for (int j = 0; j < 16; j++) {
             const int nib = j & 1;
-            // slice s has landed when only slice s + 1's loads (and at j = 0 the sums, Q5_K) are
-            // outstanding
+            // slice s has landed when only the loads of slice s + 1 (one m-tile: of s + 1 and s + 2), and at
+            // j = 0 the sums (Q5_K), are outstanding
             k8_vm<2>(k8_wait<Q5, MT>(j));
             int sc3;
             if constexpr (MT == 2) {

@@ -71,6 +71,10 @@ AETH_API int aeth_block_geometry(int dtype, int* block_elems, int* block_bytes);
  *   F32 / F16 / Q2_K / Q3_K — the GGUF tensor as the file holds it, [k][n]
  *     read as one flat run of elements / blocks (model_loader.rs:348-350);
  *     kept as is (Q2_K / Q3_K need n % 256 == 0).
+ * aeth_weight_create waits for `stream` where it reads back a flag (a block
+ * scale, or a GGUF-order F16 weight, that is infinite or NaN: Q8_0 / Q4_K / Q5_K /
+ * Q6_K / F16) and for any raw bytes on the host; F32 / Q2_K / Q3_K bytes on the
+ * device are copied in stream order.
  * aeth_weight_export_raw reproduces the original bytes. The QuantKernel
  * host-slice path registers weights implicitly (see aeth_quantized_matmul_impl). */
 typedef struct aeth_weight aeth_weight;
@@ -250,7 +254,7 @@ AETH_API int aeth_attn_decode_noalloc(const float* d_q, const float* d_layer_kv,
  * query i (row i of d_q, [n][q_stride] with head h at column h*head_dim, RoPE
  * already applied) attends to cache slots 0..i of the layer slice d_layer_kv
  * ([2][kv_heads][max_seq][head_dim]); d_out is [n][n_heads*head_dim].
- * Long prompts (from 640 tokens on at 32 / 8 heads) lay K and V out in a buffer
+ * Long prompts (from 513 tokens on at 32 / 8 heads) lay K and V out in a buffer
  * the library keeps per (device, stream), 32 KiB per KV head and 32 keys, which
  * grows on first use of a longer prompt (a grow waits for the stream). Under
  * graph capture, and where there is no memory for it, the same attention runs
