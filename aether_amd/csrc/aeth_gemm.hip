@@ -4,7 +4,7 @@
 // "Exact" mode on fp16 MFMA (v_mfma_f32_32x32x16_f16, fp32 accumulate):
 //  * A is split into two fp16 parts, A·2^-e = Ah + Al (Ah = fp16(A·2^-e),
 //    Al = fp16(A·2^-e − Ah)): 22 significant bits, f32-level. The power of two
-//    2^e is chosen per row: 0 while its largest value lies in [2^-3, 2^14), otherwise
+//    2^e is chosen per row: 0 while its largest value lies in [2, 2^14), otherwise
 //    such that it lies in [2^13, 2^14): the parts stay in fp16 range, and the lo parts
 //    of what matters to the row out of its subnormals (a row of 1e-4 unscaled keeps 13
 //    bits; a shared exponent for several rows would do the same to a small row next to
@@ -60,7 +60,7 @@
 #define G2_LOADS 6
 
 // ── activation prep (f32 A [m][k]; rows m..mp-1 read as zero). Writes
-//  * escale[r] = 2^e, e = 0 if 2^-3 <= max |A[r]| < 2^14, else the least (from −100 on)
+//  * escale[r] = 2^e, e = 0 if 2 <= max |A[r]| < 2^14, else the least (from −100 on)
 //    with |A[r]·2^-e| < 2^14. F16W, the F16 product's (a template argument: a test at run time of
 //    every element cost the other GEMMs 1.5 % of their time): always that, and −1 with zero
 //    fragments for a row that the kernel sums in f64 instead: one with an infinity, or whose largest
@@ -245,7 +245,7 @@ __global__ void __launch_bounds__(64 * PREP_ROWS * PREP_WK) k_gemm_prep(PrepArgs
     }
     int E = 14;
     if (mx > 0.0f && isfinite(mx)) (void)frexpf(mx, &E);
-    const float esc = ldexpf(1.0f, F16W || E > 14 || E < -2 ? max(E - 14, -100) : 0);
+    const float esc = ldexpf(1.0f, F16W || E > 14 || E < 2 ? max(E - 14, -100) : 0);
     const bool apart = F16W && (mx == INFINITY || ((float)(__float_as_uint(mx) >> 16) - 13 * 128.0f) * groups > logs);
     if (j == 0 && lane == 0) P.escale[r] = apart ? -1.0f : esc;
     const float inv = 1.0f / esc;  // a power of two: the products below are exact scalings

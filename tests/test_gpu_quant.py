@@ -374,12 +374,12 @@ def test_gemm_kq_one_m_tile(gpu, dtype, m, n, k):
 @pytest.mark.parametrize("dtype", [Q4_K, Q5_K, Q6_K, Q8_0])
 def test_gemm_row_exponents(gpu, dtype):
     """Rows from 2^-60 to 2^20 through the activation split of the exact-mode GEMMs, on both sides of the magnitudes where
-    a row takes a power of two (2^-3, 2^14). The parts leave 2^-22 of a value and 2^-22 of the row's largest; the sum
+    a row takes a power of two (2, 2^14). The parts leave 2^-22 of a value and 2^-22 of the row's largest; the sum
     runs through 2·k/8 products a wave and a tree; terms are bounded with the two parts of a weight that cancel."""
     m, n, k = 64, 1024, 4096
     rng = np.random.default_rng(dtype)
     x = rng.standard_normal((m, k)).astype(np.float32)
-    for i, e in enumerate((-60, -24, -13, -4, -3, -2, -1, 0, 13, 14, 20)):  # max |x[i]| = 0.75·2^e
+    for i, e in enumerate((-60, -24, -13, -4, -3, -2, -1, 0, 1, 2, 13, 14, 20)):  # max |x[i]| = 0.75·2^e
         x[i] *= np.float32(0.75 * 2.0 ** e) / np.abs(x[i]).max()
     raw = weight(dtype, n, k, 3 + dtype)
     w = make_weight(gpu, dtype, n, k, raw)
