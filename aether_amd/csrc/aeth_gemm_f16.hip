@@ -17,7 +17,7 @@
 // 4n + c, so the transpose is 16 v_perm a slice and a lane ends with four neighbouring outputs.
 // What bounds it: operand bytes, 8 KiB per wave and slice (64 B per CU and clock at the full MFMA rate; the
 // L2s deliver about a third of that). m = 333, 4096 × 4096: 456 → 40.5 µs with the prep;
-// m = 512, 14336 × 4096: 1834 → 160 µs.
+// m = 512, 14336 × 4096: 1834 → 162 µs.
 #include <math.h>
 #include <stdint.h>
 

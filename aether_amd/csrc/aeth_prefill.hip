@@ -748,11 +748,6 @@ __global__ void __launch_bounds__(512, 2) k_attn_prefill_sp(const float* __restr
     for (int t = lane; t < ntiles; t += 64) bad |= ex[t].x == SP_BAD;
     bad = __any(bad);
     if (lane < 2) far[lane][w] = 0;  // (a wave's own: no barrier; a store to LDS under the stage's loads would wait for them)
-    if (lane < 2) far[lane][w] = 0;  // (a wave's own: no barrier; a store to LDS under the stage's loads would wait for them)
-    auto plain = [&](int q0) {
-        sp_plain<G>(qkv, qkv_stride, layer_kv + (int64_t)g * max_seq * 128, layer_kv + (int64_t)(nkv + g) * max_seq * 128, n, nh,
-                    g, q0, window, out, (SpPlain*)smem);
-    };
     const uint32_t sm0 = lds_addr(smem);
     const float sl2 = 1.4426950408889634f / sqrtf(128.0f);  // scale · log2(e)
     for (int pass = 0; pass < 2; pass++) {
